@@ -653,16 +653,10 @@ __global__ __launch_bounds__(256) void k_near_apply(const int2 *__restrict__ til
 // The plain form's nearfield without the coefficient stream: at q = 1 every
 // source but the panel itself by KER = A_x A_y ker4(p_x - p_y) in FP64, plus
 // the stored corrections (rule minus formula) of the self / shared-vertex
-// pairs.  Same tiles as k_near_apply; sources (p, A sigma), (n, A sigma_n)
-// staged in LDS.  The values differ from the stored coefficients only by the
-// rounding of the formula's operation order.
-#define FLY64_CHUNK 512
-#define FLY64_RB 2   // rows per pass over the staged sources
-#define FLY64_OWNSPLIT 1   // the self-pair selects only on the tile's own leaf columns
-// TR: the transposed operator's row x, i.e. KER(y, x) read transposed: with
-// r, n_x, n_y as below, y0 and y3 are symmetric in (x, y) and
-//   y1(y,x) = -(eps coef - 1) dG0dx,  y2(y,x) = -(coef/eps - 1) dG0dy,
-//   out[x] += y3 A sgm_n + y1(y,x) A sgm,  out[x+n] += y2(y,x) A sgm_n + y0 A sgm
+// pairs.  Same tiles as k_near_apply.  The values differ from the stored
+// coefficients only by the rounding of the formula's operation order.
+#define FLY64_CHUNK 512   // staged source columns per pass
+#define FLY64_TAB 1024    // LDS entries of e^{-kappa r} at equal steps of r (NearK)
 // 1/sqrt(x) for x > 0 (a normal FP64 number): the hardware estimate (relative
 // error 2^-24 measured on gfx950), then one third-order step
 // y <- y (1 + e/2 + 3e^2/8), e = 1 - x y^2, which cubes the error (measured
@@ -695,141 +689,187 @@ __global__ void k_exp2_tab() {
   if (j < 256) gExp2Tab[j] = exp2((double)j / 256.0);
 }
 
-// One pair of the on-the-fly FP64 nearfield (kernelKER4 at the one-point rule,
-// src/kernel.c:109-147): target point/normal X, XN against staged source
-// P = (point, A sigma), N = (normal, A sigma_n).  skip: the panel itself (its
-// weights are zeroed and r2 replaced by 1 so nothing divides by zero).
-// CHK: the source may be the panel itself (the tile's own leaf columns).
-// Every term is linear in G0 = 1/(4 pi r), so the sums are kept with G0
-// replaced by 1/r and the row's total is scaled by 1/(4 pi) once; with
-// a = ipX dG0dy shared by ddG0 and the kappa^2 term, and the accumulations as
-// FMA chains, a pair is 60 FP64/integer VALU instructions.
-template <bool TR, bool CHK>
-__device__ __forceinline__ void fly64Pair(const double4 &X, const double4 &XN, const double4 &P, const double4 &N,
-                                          bool skip, double kappa, double kap2, double eps, double ieps,
-                                          const double *__restrict__ T, double &s0, double &s1) {
-  const double rx = X.x - P.x, ry = X.y - P.y, rz = X.z - P.z;
+// Constants of the on-the-fly FP64 nearfield.  With q the scalar density (A
+// sigma_n; transposed A sigma), m = 3 n_y times the other one, r = x - y,
+// B = (coef - 1)/r^3, e = e^{-kappa r}, coef = (kappa r + 1) e, every term of a
+// row is one of five sums over its sources,
+//   F = sum q' (1 - e)/r,  S1 = sum B (m.r),  S2 = sum (m.r)/r^3,
+//   R = sum [q' (B + cc/r^3) - (m.r)(B/r^2 + (kappa^2/3) e/r^3)] r,  N = sum B m,
+// with q' = qs q, and the row's two values are
+//   fF F + f1 S1 + f2 S2  and  n_x . (R + N/3)
+// (kernelKER4, src/kernel.c:109-147, at the one-point rule; the factors A_x/4pi
+// and n_x leave the source loop).  The transposed operator's row is the same
+// with the densities' roles exchanged, 1/eps for eps and the sign of the terms
+// odd in r flipped: y1(y,x) = -(eps coef - 1) dG0dx, y2(y,x) = -(coef/eps - 1) dG0dy.
+struct NearK {
+  double kappa, k23, cc, qs, fF, f1, f2;
+  // e^{-kappa r} = T[k] P(r - k h), k = rint(r / h), kappa h = 1/256: T in LDS, P the
+  // degree-4 Taylor polynomial economised on |z| <= 1/512 (the z^5/120 term
+  // replaced by its Chebyshev remainder: truncation h^5/1920 = 1.5e-17)
+  double h, invh, p1, p2, p3, p4;
+  int nT;   // entries of T (0: the largest near distance needs more; e by expNeg)
+};
+
+// one tile of the launch order, everything a block needs in one load
+struct NearTile {
+  int row0, rows;        // destination panels
+  int src, ncol;         // its leaf's columns in the source list
+  int own, nOwn, tile;   // the leaf's own columns; the tile's number
+  int pad;
+};
+
+struct NearAcc {
+  double F, S1, S2, rx, ry, rz, nx, ny, nz;
+};
+
+// One pair: target point (X, Y, Z) against staged source P = (point, q') and m.
+// 44 FP64 instructions and the reciprocal square root (of which 9 for e^{-kappa r}
+// from the table of steps; expNeg 15).  skip: the panel itself (its weights are
+// zeroed and r2 replaced by 1 so nothing divides by zero).  CHK: the source may
+// be the panel itself (the tile's own leaf columns).  TAB: NearK's table.
+template <bool CHK, bool TAB>
+__device__ __forceinline__ void fly64Pair(double X, double Y, double Z, const double4 &P, double mx, double my,
+                                          double mz, bool skip, const NearK &K, const double *__restrict__ T,
+                                          NearAcc &a) {
+  const double rx = X - P.x, ry = Y - P.y, rz = Z - P.z;
   const double r2 = CHK && skip ? 1.0 : rx * rx + ry * ry + rz * rz;
-  const double ri = rsq64(r2), rn = r2 * ri, ri2 = ri * ri, ri3 = ri * ri2;
-  const double kr = kappa * rn;
-  const double e = expNeg(-kr, T);
-  const double ip0 = XN.x * N.x + XN.y * N.y + XN.z * N.z;
-  const double ipX = XN.x * rx + XN.y * ry + XN.z * rz;
-  const double ipY = N.x * rx + N.y * ry + N.z * rz;
-  // 4 pi times: G0, dG0/dn_y, dG0/dn_x, d2G0/dn_x dn_y
-  const double coef = (kr + 1.0) * e;
-  const double dy = ipY * ri3, dx = ipX * ri3;
-  const double a = ipX * dy;
-  const double ddG = fma(a * ri2, -3.0, ip0 * ri3);
-  const double y0 = fma(-ri, e, ri);
-  const double y3 = fma(coef, ddG, -(kap2 * e) * a) - ddG;
-  const double pw = CHK && skip ? 0.0 : P.w, nw = CHK && skip ? 0.0 : N.w;
-  if constexpr (TR) {
-    const double y1 = fma(-eps, coef * dx, dx);
-    const double y2 = fma(-(coef * dy), ieps, dy);
-    s0 = fma(y3, nw, fma(y1, pw, s0));
-    s1 = fma(y2, nw, fma(y0, pw, s1));
+  const double y = __builtin_amdgcn_rsq(r2), t = r2 * y;   // rsq64's step, which also gives r = r2 / r
+  const double er = fma(-t, y, 1.0), q = er * fma(er, 0.375, 0.5);
+  const double ri = fma(y, q, y), rn = fma(t, q, t);
+  const double kr = K.kappa * rn;
+  double e;
+  if constexpr (TAB) {
+    const double u = fma(rn, K.invh, 0x1.8p52);   // rint(r / h) in the low word
+    const double d = fma(u - 0x1.8p52, -K.h, rn);
+    e = T[__double2loint(u)] * fma(d, fma(d, fma(d, fma(d, K.p4, K.p3), K.p2), K.p1), 1.0);
   } else {
-    const double y1 = fma(eps, coef * dy, -dy);
-    const double y2 = fma(coef * dx, ieps, -dx);
-    s0 = fma(y0, nw, fma(y1, pw, s0));
-    s1 = fma(y2, nw, fma(y3, pw, s1));
+    e = expNeg(-kr, T);
   }
+  const double ri2 = ri * ri, q3 = ri * ri2;
+  const double ip = fma(mx, rx, fma(my, ry, mz * rz));
+  const double B = fma(fma(kr, e, e), q3, -q3);
+  const double w = CHK && skip ? 0.0 : P.w, im = CHK && skip ? 0.0 : ip, Bn = CHK && skip ? 0.0 : B;
+  a.F = fma(fma(-ri, e, ri), w, a.F);
+  a.S1 = fma(B, im, a.S1);
+  a.S2 = fma(q3, im, a.S2);
+  const double W = fma(ri2, B, (K.k23 * e) * q3);
+  const double A = fma(w, fma(K.cc, q3, B), -(im * W));
+  a.rx = fma(A, rx, a.rx);
+  a.ry = fma(A, ry, a.ry);
+  a.rz = fma(A, rz, a.rz);
+  a.nx = fma(Bn, mx, a.nx);
+  a.ny = fma(Bn, my, a.ny);
+  a.nz = fma(Bn, mz, a.nz);
 }
 
-// Staged columns [j0, j1) against the wave's rows h .. h + FLY64_RB - 1, one
-// column per lane (rows past the tile skipped wave-uniformly).  CHK: the
-// columns may hold the row's own panel.  The own leaf's columns run as a
-// range of their own so that no pass executes both forms under a split
-// lane mask.
-template <bool TR, bool CHK>
-__device__ __forceinline__ void fly64Cols(int h, int j0, int j1, int lane, int w, int rows, const double4 *sP,
-                                          const double4 *sN, const int *sY, const double4 (&X)[FLY64_RB],
-                                          const double4 (&XN)[FLY64_RB], const int (&xi)[4], double kappa,
-                                          double kap2, double eps, double ieps, const double *__restrict__ T,
-                                          double (&a0)[4], double (&a1)[4]) {
+// Staged columns [j0, j1) against the wave's four rows, one column per lane
+// (rows past the tile skipped wave-uniformly; the rows' points are
+// wave-uniform, so they sit in scalar registers).  CHK: the columns may hold
+// the row's own panel.  The own leaf's columns run as a range of their own so
+// that no pass executes both forms under a split lane mask.
+template <bool CHK, bool TAB>
+__device__ __forceinline__ void fly64Cols(int j0, int j1, int lane, int w, int rows, const double4 *sP,
+                                          const double2 *sM, const double *sMz, const int *sY,
+                                          const double (&X)[4][3], const int (&xi)[4], const NearK &K,
+                                          const double *__restrict__ T, NearAcc (&acc)[4]) {
   for (int j = j0 + lane; j < j1; j += 64) {
-    const double4 P = sP[j], N = sN[j];
+    const double4 P = sP[j];
+    const double2 M = sM[j];
+    const double mz = sMz[j];
     const int y = CHK ? sY[j] : -1;
 #pragma unroll
-    for (int r = 0; r < FLY64_RB; r++)
-      if (w + 4 * (h + r) < rows)
-        fly64Pair<TR, CHK>(X[r], XN[r], P, N, CHK && y == xi[h + r], kappa, kap2, eps, ieps, T, a0[h + r],
-                           a1[h + r]);
+    for (int r = 0; r < 4; r++)
+      if (w + 4 * r < rows)
+        fly64Pair<CHK, TAB>(X[r][0], X[r][1], X[r][2], P, M.x, M.y, mz, CHK && y == xi[r], K, T, acc[r]);
   }
 }
 
-template <bool TR>
-__device__ __forceinline__ void nearFly64Tile(int t, const int2 *__restrict__ tiles,
-                                              const int *__restrict__ leafStart, const int *__restrict__ leafCount,
-                                              const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
-                                              const int *__restrict__ srcList, const double4 *__restrict__ PA,
-                                              const double4 *__restrict__ PN, const double *__restrict__ x,
-                                              const long long *__restrict__ specOff, const int *__restrict__ specCol,
-                                              const double4 *__restrict__ specVal, double *__restrict__ out, int n,
-                                              double kappa, double eps, double4 *sP, double4 *sN, int *sY,
-                                              double *sE, const int *__restrict__ ownOff) {
-  const int2 tl = tiles[t];
-  const int D = tl.x, r0 = tl.y;
-  const int oc = ownOff[D], nOwn = oc >= 0 ? leafCount[D] : 0;   // D's own columns: [oc, oc + nOwn)
-  const int rows = min(NEAR_ROWS, leafCount[D] - r0);
-  const int ncol = ncolArr[D];
-  const int *src = srcList + srcOff[D];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const double ieps = 1.0 / eps, kap2 = kappa * kappa;
-  // wave w owns rows w, w + 4, w + 8, w + 12 and takes each staged source once
-  // for FLY64_RB of them at a time, held in registers (rows past the tile are
-  // skipped wave-uniformly)
+// FP64 issue bounds it (the card sustains 2.8e13 FP64 lane instructions per
+// second, 72 % of its nominal clock's rate), so the split aims at the fewest
+// instructions per pair: wave w owns rows w, w + 4, w + 8, w + 12 and takes each
+// staged source (56 bytes of LDS) once for all four, their nine sums in
+// registers.  317k panels, alone: 988 us with kernelKER4's operation order, two
+// rows per pass and the corrections added row by row at the end; 1,078 us with
+// these sums but the corrections still there; 788 us so (81,920 panels: 262 ->
+// 212 us).  On a bare copy of the loop (3.9e8 pairs): four rows 769 us, two 809,
+// one 923; without the per-row test (the pairs interleaved, 229 VGPRs) 884; at
+// four waves per SIMD 923 (29 spills).
+template <bool TAB>
+__device__ __forceinline__ void nearFly64Tile(const NearTile &tl, const int *__restrict__ srcList,
+                                              const double4 *__restrict__ PA, const double4 *__restrict__ PN,
+                                              const double *__restrict__ x, const long long *__restrict__ specOff,
+                                              const int *__restrict__ specCol, const double4 *__restrict__ specVal,
+                                              double *__restrict__ out, int n, const NearK &K, int tr, double4 *sP,
+                                              double2 *sM, double *sMz, int *sY, const double *sE) {
+  const int oc = tl.own, nOwn = tl.nOwn, rows = tl.rows, ncol = tl.ncol;   // own columns: [oc, oc + nOwn)
+  const int *src = srcList + tl.src;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int oS = tr ? 0 : n, oM = tr ? n : 0;   // where the scalar density and the one on n_y sit in x
   int xi[4];
 #pragma unroll
-  for (int r = 0; r < 4; r++) xi[r] = leafStart[D] + r0 + min(w + 4 * r, rows - 1);
-  double a0[4] = {0, 0, 0, 0}, a1[4] = {0, 0, 0, 0};
+  for (int r = 0; r < 4; r++) xi[r] = tl.row0 + min(w + 4 * r, rows - 1);
+  NearAcc acc[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) acc[r] = NearAcc{0, 0, 0, 0, 0, 0, 0, 0, 0};
+  // the rows' stored corrections first, sixteen lanes a row, so that their chain of
+  // loads runs under the other waves' arithmetic instead of at the tile's end, row
+  // after row
+  double cor0 = 0.0, cor1 = 0.0;
+  {
+    const int row = w + 4 * (lane >> 4), xr = tl.row0 + min(row, rows - 1);
+    const long long e1 = row < rows ? specOff[xr + 1] : 0;
+    for (long long e = specOff[xr] + (lane & 15); e < e1; e += 16) {
+      const int y = specCol[e];
+      const double4 d = specVal[e];
+      const double p = x[y], m = x[y + n];
+      cor0 += d.x * m + d.y * p;
+      cor1 += d.z * m + d.w * p;
+    }
+  }
   for (int c0 = 0; c0 < ncol; c0 += FLY64_CHUNK) {
     const int cn = min(FLY64_CHUNK, ncol - c0);
     __syncthreads();
     for (int j = threadIdx.x; j < cn; j += 256) {
       const int y = src[c0 + j];
       const double4 p = PA[y], nn = PN[y];
-      sP[j] = make_double4(p.x, p.y, p.z, p.w * x[y]);
-      sN[j] = make_double4(nn.x, nn.y, nn.z, p.w * x[y + n]);
+      const double m = 3.0 * p.w * x[y + oM];
+      sP[j] = make_double4(p.x, p.y, p.z, K.qs * p.w * x[y + oS]);
+      sM[j] = make_double2(nn.x * m, nn.y * m);
+      sMz[j] = nn.z * m;
       sY[j] = y;
     }
     __syncthreads();
+    if (w < rows) {
+      double X[4][3];
 #pragma unroll
-    for (int h = 0; h < 4; h += FLY64_RB) {
-      if (w + 4 * h >= rows) break;
-      double4 X[FLY64_RB], XN[FLY64_RB];
-#pragma unroll
-      for (int r = 0; r < FLY64_RB; r++) {
-        X[r] = PA[xi[h + r]];
-        XN[r] = PN[xi[h + r]];
+      for (int r = 0; r < 4; r++) {
+        const double4 p = PA[xi[r]];
+        X[r][0] = p.x;
+        X[r][1] = p.y;
+        X[r][2] = p.z;
       }
-      if (FLY64_OWNSPLIT) {   // D's own columns [lo, hi) of this chunk apart, each range a loop of its own;
-        // the checked range is extended to whole passes of 64 columns (the check
-        // is exact for any column), so it leaves no partly idle pass behind
-        const int lo = min(max(oc - c0, 0), cn);
-        const int hi = min(lo + ((min(max(oc + nOwn - c0, 0), cn) - lo + 63) & ~63), cn);
-        fly64Cols<TR, false>(h, 0, lo, lane, w, rows, sP, sN, sY, X, XN, xi, kappa, kap2, eps, ieps, sE, a0, a1);
-        fly64Cols<TR, true>(h, lo, hi, lane, w, rows, sP, sN, sY, X, XN, xi, kappa, kap2, eps, ieps, sE, a0, a1);
-        fly64Cols<TR, false>(h, hi, cn, lane, w, rows, sP, sN, sY, X, XN, xi, kappa, kap2, eps, ieps, sE, a0, a1);
-      } else {
-        fly64Cols<TR, true>(h, 0, cn, lane, w, rows, sP, sN, sY, X, XN, xi, kappa, kap2, eps, ieps, sE, a0, a1);
-      }
+      // D's own columns [lo, hi) of this chunk apart, each range a loop of its own;
+      // the checked range is extended to whole passes of 64 columns (the check
+      // is exact for any column), so it leaves no partly idle pass behind
+      const int lo = min(max(oc - c0, 0), cn);
+      const int hi = min(lo + ((min(max(oc + nOwn - c0, 0), cn) - lo + 63) & ~63), cn);
+      fly64Cols<false, TAB>(0, lo, lane, w, rows, sP, sM, sMz, sY, X, xi, K, sE, acc);
+      fly64Cols<true, TAB>(lo, hi, lane, w, rows, sP, sM, sMz, sY, X, xi, K, sE, acc);
+      fly64Cols<false, TAB>(hi, cn, lane, w, rows, sP, sM, sMz, sY, X, xi, K, sE, acc);
     }
   }
+#pragma unroll
   for (int r = 0; r < 4; r++) {
     const int row = w + 4 * r;
     const double A = PA[xi[r]].w * kFourPiI;
-    double t0 = A * a0[r], t1 = A * a1[r];
-    if (row < rows)
-      for (long long e = specOff[xi[r]] + lane; e < specOff[xi[r] + 1]; e += 64) {
-        const int y = specCol[e];
-        const double4 d = specVal[e];
-        t0 += d.x * x[y + n] + d.y * x[y];
-        t1 += d.z * x[y + n] + d.w * x[y];
-      }
-    t0 = waveSumT(t0);
-    t1 = waveSumT(t1);
+    const double4 N = PN[xi[r]];
+    const NearAcc &s = acc[r];
+    const double sS = A * (K.fF * s.F + K.f1 * s.S1 + K.f2 * s.S2);
+    const double sV = A * (N.x * (s.rx + s.nx * (1.0 / 3)) + N.y * (s.ry + s.ny * (1.0 / 3)) +
+                           N.z * (s.rz + s.nz * (1.0 / 3)));
+    const bool mine = (lane >> 4) == r;
+    const double t0 = waveSumT((tr ? sV : sS) + (mine ? cor0 : 0.0));
+    const double t1 = waveSumT((tr ? sS : sV) + (mine ? cor1 : 0.0));
     if (row < rows && lane == 0) {
       out[xi[r]] = t0;
       out[xi[r] + n] = t1;
@@ -837,43 +877,49 @@ __device__ __forceinline__ void nearFly64Tile(int t, const int2 *__restrict__ ti
   }
 }
 
-// The mixed nearfield: tiles with a stored coefficient block (tileCoef >= 0)
-// stream it (HBM-bound), the others compute their pairs on the fly
-// (VALU-bound).  The host interleaves the two kinds in block order, so every
-// CU holds both at once and the stream and the arithmetic overlap.
-#define MIX64_LDS (2 * FLY64_CHUNK * 32 + FLY64_CHUNK * 4)
-static_assert(MIX64_LDS >= 2 * NEAR_CHUNK * 8, "the stream tiles' LDS must fit the union");
-template <bool TR = false>
-__global__ __launch_bounds__(256) void k_near_mix64(const int2 *__restrict__ tiles, const int *__restrict__ leafStart,
-                                                    const int *__restrict__ leafCount,
-                                                    const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
-                                                    const long long *__restrict__ tileCoef,
-                                                    const int *__restrict__ srcList,
-                                                    const double4 *__restrict__ coef, const double4 *__restrict__ PA,
-                                                    const double4 *__restrict__ PN, const double *__restrict__ x,
-                                                    const long long *__restrict__ specOff,
-                                                    const int *__restrict__ specCol,
-                                                    const double4 *__restrict__ specVal, double *__restrict__ out,
-                                                    int n, double kappa, double eps, int nTiles,
-                                                    const int *__restrict__ order, const int *__restrict__ ownOff) {
-  __shared__ __align__(16) unsigned char lds[MIX64_LDS];
-  __shared__ double sE[256];   // 2^(j/256) for expNeg
-  for (int j = threadIdx.x; j < 256; j += blockDim.x) sE[j] = gExp2Tab[j];
-  // tiles in `order`, costliest first (the default grid has one block per tile;
-  // a smaller grid strides over them)
-  for (int k = blockIdx.x; k < nTiles; k += gridDim.x) {
-    const int t = order[k];
-    __syncthreads();
-    if (tileCoef[t] >= 0) {
-      double *sS = reinterpret_cast<double *>(lds);
-      nearStreamTile<double>(t, tiles, leafStart, leafCount, srcOff, ncolArr, tileCoef, srcList, coef, x, out, n, sS,
-                             sS + NEAR_CHUNK);
-    } else {
-      double4 *sP = reinterpret_cast<double4 *>(lds);
-      nearFly64Tile<TR>(t, tiles, leafStart, leafCount, srcOff, ncolArr, srcList, PA, PN, x, specOff, specCol,
-                        specVal, out, n, kappa, eps, sP, sP + FLY64_CHUNK, reinterpret_cast<int *>(sP + 2 * FLY64_CHUNK),
-                        sE, ownOff);
+// The FP64 nearfield at q = 1.  MIX: tiles with a stored coefficient block
+// (tileCoef >= 0) stream it (HBM-bound), the others compute their pairs on the
+// fly (VALU-bound); the host interleaves the two kinds in block order, so every
+// CU holds both at once and the stream and the arithmetic overlap, and a grid
+// smaller than the tiles strides over them.  Without MIX every tile is computed
+// and has a block of its own: the launch of the default configuration, which
+// needs the registers of the mixed form's other branch (171 against 151 VGPRs)
+// for its third wave per SIMD.  Tiles costliest first (desc).
+// TAB: e^{-kappa r} from NearK's table (tab, K.nT entries), else from 2^(j/256)
+// and expNeg.  tr: the transposed operator's rows.
+#define MIX64_LDS (2 * NEAR_CHUNK * 8)
+#define FLY64_LDS (FLY64_CHUNK * (32 + 16 + 8 + 4))
+static_assert(MIX64_LDS >= FLY64_LDS, "the computed tiles' LDS must fit the union");
+template <bool TAB, bool MIX>
+__global__ __launch_bounds__(256, 3) void k_near_mix64(
+    const NearTile *__restrict__ desc, const int2 *__restrict__ tiles, const int *__restrict__ leafStart,
+    const int *__restrict__ leafCount, const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
+    const long long *__restrict__ tileCoef, const int *__restrict__ srcList, const double4 *__restrict__ coef,
+    const double4 *__restrict__ PA, const double4 *__restrict__ PN, const double *__restrict__ x,
+    const long long *__restrict__ specOff, const int *__restrict__ specCol, const double4 *__restrict__ specVal,
+    double *__restrict__ out, int n, NearK K, const double *__restrict__ tab, int tr, int nTiles) {
+  __shared__ __align__(16) unsigned char lds[MIX ? MIX64_LDS : FLY64_LDS];
+  __shared__ double sE[TAB ? FLY64_TAB : 256];
+  for (int j = threadIdx.x; j < (TAB ? K.nT : 256); j += blockDim.x) sE[j] = TAB ? tab[j] : gExp2Tab[j];
+  double4 *sP = reinterpret_cast<double4 *>(lds);
+  double2 *sM = reinterpret_cast<double2 *>(sP + FLY64_CHUNK);
+  double *sMz = reinterpret_cast<double *>(sM + FLY64_CHUNK);
+  int *sY = reinterpret_cast<int *>(sMz + FLY64_CHUNK);
+  if constexpr (MIX) {
+    for (int k = blockIdx.x; k < nTiles; k += gridDim.x) {
+      const NearTile tl = desc[k];
+      __syncthreads();
+      if (tileCoef[tl.tile] >= 0) {
+        double *sS = reinterpret_cast<double *>(lds);
+        nearStreamTile<double>(tl.tile, tiles, leafStart, leafCount, srcOff, ncolArr, tileCoef, srcList, coef, x, out,
+                               n, sS, sS + NEAR_CHUNK);
+      } else {
+        nearFly64Tile<TAB>(tl, srcList, PA, PN, x, specOff, specCol, specVal, out, n, K, tr, sP, sM, sMz, sY, sE);
+      }
     }
+  } else {
+    nearFly64Tile<TAB>(desc[blockIdx.x], srcList, PA, PN, x, specOff, specCol, specVal, out, n, K, tr, sP, sM, sMz,
+                       sY, sE);
   }
 }
 
@@ -4120,6 +4166,9 @@ struct fbh_ctx {
   // FP64 nearfield on the fly (q = 1): panel data and the corrections in FP64
   bool fly64 = false;
   double4 *fly64PA = nullptr, *fly64PN = nullptr, *specVal64 = nullptr, *specValT64 = nullptr;
+  NearK nearK[2] = {};          // its constants: the operator's rows and the transposed ones
+  NearTile *nearDesc = nullptr; // its tiles in launch order
+  double *nearTab = nullptr;    // e^{-kappa r} at the steps of NearK
   double *ro = nullptr, *dx = nullptr;   // refinement residual and correction
   ChargeSet csCall;   // charge set of the calls that pass host charge arrays
   ChargeSet csRes;    // resident charge set (fbh_set_charges)
@@ -4703,7 +4752,7 @@ static inline int blk64(int n, int cap) {
   return std::max(64, std::min(b, cap));
 }
 
-static int enableFly64(fbh_ctx *c);
+static int enableFly64(fbh_ctx *c, double rMax);
 static int resolveScratch(int dev);
 
 extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorder, int n, const double *vtx,
@@ -4877,7 +4926,14 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
       cost[t] = (long long)std::min(NEAR_ROWS, leafCount[tiles[t].x] - tiles[t].y) * ncol[tiles[t].x];
     }
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-    if (!(c->tileOrder = dupload(c, order.data(), order.size())) || !(c->ownOff = dupload(c, ownOff.data(), ownOff.size())))
+    std::vector<NearTile> desc(tiles.size());
+    for (size_t k = 0; k < tiles.size(); k++) {
+      const int t = order[k], D = tiles[t].x, r0 = tiles[t].y;
+      desc[k] = {leafStart[D] + r0, std::min(NEAR_ROWS, leafCount[D] - r0), srcOff[D], ncol[D], std::max(ownOff[D], 0),
+                 ownOff[D] >= 0 ? leafCount[D] : 0, t, 0};
+    }
+    if (!(c->tileOrder = dupload(c, order.data(), order.size())) || !(c->ownOff = dupload(c, ownOff.data(), ownOff.size())) ||
+        !(c->nearDesc = dupload(c, desc.data(), desc.size())))
       FAIL();
     // blocks of the FP64 nearfield launch (0: one per tile, the fastest here;
     // resident grids of 2-4 blocks per CU were slower beside the far chain)
@@ -4968,7 +5024,31 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
     if (hipGetLastError() != hipSuccess) { setErr("k_m2l_derivs launch failed"); FAIL(); }
   }
   if (hipStreamSynchronize(c->stream) != hipSuccess) { setErr("setup kernels failed: %s", hipGetErrorString(hipGetLastError())); FAIL(); }
-  if (c->nFlyTiles > 0 && !enableFly64(c)) FAIL();
+  if (c->nFlyTiles > 0) {
+    // the largest distance between quadrature points of a near pair, bounded by the
+    // leaves' spheres about their cube centres
+    std::vector<double> rad(nLeaf, 0.0);
+    const double t = c->Q.t[0];
+    bool ok = true;
+    for (int l = 0; l < nLeaf; l++)
+      for (int j = leafStart[l]; j < leafStart[l] + leafCount[l]; j++) {
+        double d2 = 0.0;
+        for (int k = 0; k < 3; k++) {
+          const double d = hp[j].v[k] + t * (hp[j].a[6 + k] + t * hp[j].a[k]) - cubeX[3 * l + k];
+          d2 += d * d;
+        }
+        if (!std::isfinite(d2)) ok = false;
+        rad[l] = std::max(rad[l], std::sqrt(d2));
+      }
+    double rMax = 1.0;   // a panel against itself is evaluated at r = 1 with zero weight
+    for (int l = 0; l < nLeaf; l++)
+      for (int k = nearOff[l]; k < nearOff[l + 1]; k++) {
+        const double *a = &cubeX[3 * l], *b = &cubeX[3 * nearSrc[k]];
+        rMax = std::max(rMax, std::sqrt((a[0] - b[0]) * (a[0] - b[0]) + (a[1] - b[1]) * (a[1] - b[1]) +
+                                        (a[2] - b[2]) * (a[2] - b[2])) + rad[l] + rad[nearSrc[k]]);
+      }
+    if (!enableFly64(c, ok ? rMax * (1.0 + 1e-12) : HUGE_VAL)) FAIL();
+  }
 #undef FAIL
   return c;
 }
@@ -5155,14 +5235,30 @@ static void farPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_t
   l2pPass(c, B, st);
 }
 
+// The FP64 mixed nearfield of the operator (tr 0) or its transpose into c->nearv.
+// e^{-kappa r} comes from the table of steps wherever the near distances fit its
+// FLY64_TAB entries (kappa r up to 4: every leaf size in use); beyond it expNeg.
+static void nearMix64(fbh_ctx *c, const double4 *coef, const double4 *spec, const double *x, int tr, hipStream_t st) {
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(c->nearGrid), dim3(256), 0, st, c->nearDesc, c->tiles, c->leafStart, c->leafCount,
+                       c->srcOff, c->ncol, c->tileCoef, c->srcList, coef, c->fly64PA, c->fly64PN, x, c->specOff,
+                       c->specCol, spec, c->nearv, c->n, c->nearK[tr], c->nearTab, tr, c->nTiles);
+  };
+  const bool mix = c->nStored > 0 || c->nearGrid < c->nTiles;
+  if (c->nearK[tr].nT > 0) {
+    if (mix) launch(k_near_mix64<true, true>);
+    else launch(k_near_mix64<true, false>);
+  } else {
+    if (mix) launch(k_near_mix64<false, true>);
+    else launch(k_near_mix64<false, false>);
+  }
+}
+
 template <typename R>
 static void nearPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_t st) {
   if (c->nFlyTiles > 0) {
     if constexpr (std::is_same<R, double>::value)
-      hipLaunchKernelGGL(k_near_mix64<false>, dim3(c->nearGrid), dim3(256), 0, st, c->tiles, c->leafStart,
-                         c->leafCount, c->srcOff, c->ncol, c->tileCoef, c->srcList, B.coef, c->fly64PA, c->fly64PN, x,
-                         c->specOff, c->specCol, c->specVal64, B.nearv, c->n, c->kappa, c->eps, c->nTiles,
-                         c->tileOrder, c->ownOff);
+      nearMix64(c, B.coef, c->specVal64, x, 0, st);
     else
       hipLaunchKernelGGL(k_near_mix32, dim3(c->nTiles), dim3(256), c->near32Pad, st, c->tiles, c->leafStart, c->leafCount,
                          c->srcOff, c->ncol, c->tileCoef, c->srcList, B.coef, c->flyPA, c->flyPN, c->flyPL, x,
@@ -5288,10 +5384,7 @@ static int matvecTr(fbh_ctx *c, double alpha, const double *x, double beta, doub
   HCK(hipEventRecord(c->evFork, c->stream));
   HCK(hipStreamWaitEvent(c->side, c->evFork, 0));
   if (c->nFlyTiles > 0)
-    hipLaunchKernelGGL(k_near_mix64<true>, dim3(c->nearGrid), dim3(256), 0, c->side, c->tiles, c->leafStart,
-                       c->leafCount, c->srcOff, c->ncol, c->tileCoef, c->srcList, c->coefT, c->fly64PA, c->fly64PN, x,
-                       c->specOff, c->specCol, c->specValT64, c->nearv, c->n, c->kappa, c->eps, c->nTiles,
-                       c->tileOrder, c->ownOff);
+    nearMix64(c, c->coefT, c->specValT64, x, 1, c->side);
   else
     hipLaunchKernelGGL(k_near_apply<double>, dim3(c->nTiles), dim3(256), 0, c->side, c->tiles, c->leafStart,
                        c->leafCount, c->srcOff, c->ncol, c->tileCoef, c->srcList, c->coefT, x, c->nearv, c->n);
@@ -5335,9 +5428,36 @@ static int ensureSpec(fbh_ctx *c) {
   return 1;
 }
 
-// panel data and special-pair corrections of the tiles computed on the fly
-static int enableFly64(fbh_ctx *c) {
+// panel data, kernel constants and special-pair corrections of the tiles computed on
+// the fly; rMax bounds the near distances
+static int enableFly64(fbh_ctx *c, double rMax) {
   const size_t n = c->n;
+  NearK K{};
+  const double ka = c->kappa;
+  K.kappa = ka;
+  K.k23 = ka * ka / 3.0;
+  K.h = ka != 0.0 ? std::min(1.0 / (256.0 * std::fabs(ka)), rMax) : rMax;
+  if (std::isfinite(rMax) && rMax / K.h <= FLY64_TAB - 3) {
+    K.invh = 1.0 / K.h;
+    K.nT = (int)std::ceil(rMax * K.invh) + 2;
+    const double w = 0.5 * ka * K.h;   // half width of a step in kappa r (even powers only)
+    K.p1 = ka * (-1.0 + w * w * w * w / 384.0);
+    K.p2 = ka * ka / 2.0;
+    K.p3 = ka * ka * ka * (-1.0 / 6.0 - w * w / 96.0);
+    K.p4 = ka * ka * ka * ka / 24.0;
+    std::vector<double> T(K.nT);
+    for (int k = 0; k < K.nT; k++) T[k] = std::exp(-ka * K.h * k);
+    if (!(c->nearTab = dupload(c, T.data(), T.size()))) return 0;
+  }
+  for (int tr = 0; tr < 2; tr++) {
+    const double e = tr ? 1.0 / c->eps : c->eps, sg = tr ? -1.0 : 1.0;
+    NearK &o = c->nearK[tr] = K;
+    o.qs = sg / e;
+    o.cc = 1.0 - e;
+    o.fF = sg * e;
+    o.f1 = sg * e / 3.0;
+    o.f2 = sg * (e - 1.0) / 3.0;
+  }
   if (!(c->fly64PA = dalloc<double4>(c, n)) || !(c->fly64PN = dalloc<double4>(c, n)) || !ensureSpec(c) ||
       !(c->specVal64 = dalloc<double4>(c, (size_t)c->nSpec)))
     return 0;

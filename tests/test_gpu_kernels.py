@@ -1,0 +1,46 @@
+"""Kernels chosen by a rule on sizes or parameters, on both sides of the rule and at
+its edges, against the oracle (FP64 bar of the parity tests: 1e-13 relative)."""
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle_binding as O
+from conftest import ROOT, rel
+
+pytestmark = pytest.mark.gpu
+_meshes = {}
+
+
+def molecule(fa, tmp_path_factory, kind, level, radius, *extra):
+    key = (kind, level, radius) + extra
+    if key not in _meshes:
+        base = str(tmp_path_factory.mktemp("mesh") / "m")
+        subprocess.check_call([f"{ROOT}/cuda-fabipb_amd/bin/fbmesh", kind, base, "--level", str(level), "--radius",
+                               str(radius), *extra], stdout=subprocess.DEVNULL)
+        _meshes[key] = fa.Mesh(base)
+    return _meshes[key]
+
+
+GLOBULE = ("--charges", "inside", "--nq", "40", "--sigma", "0.4", "--depth", "1.5", "--seed", "9", "--merge", "0.45")
+
+
+@pytest.mark.parametrize("kappa,depth", [(0.0, 2), (1e-4, 2), (0.1257, 2), (0.1257, 1), (0.3, 1), (2.5, 2)])
+def test_near_exponential_table(fa, tmp_path_factory, kappa, depth):
+    """The nearfield's table of e^{-kappa r} (kappa times the near distances up to 4) and
+    the general form beyond it; leaves whose row count leaves every remainder of a tile."""
+    mesh = molecule(fa, tmp_path_factory, "globule", 3, 8, *GLOBULE)
+    tree = fa.Tree(mesh, depth, order=6, height=min(2, depth))
+    op = fa.Operator(tree, kappa, 1.0, 80.0, 1)
+    x, y = np.random.default_rng(1).uniform(-1, 1, (2, 2 * tree.n))
+    ora = O.Oracle(tree.oracle_layout(kappa, 1.0, 80.0, 1))
+    ax = op.matvec(x)
+    assert rel(ax, ora.matvec(x)) <= 1e-13
+    if op.stats()["m2l_pairs"] == 0:   # one level: the adjoint operator needs M2L tensors
+        return
+    import torch
+    yd = torch.tensor(y, device="cuda")
+    at = torch.empty_like(yd)
+    op.matvec_t_dev(yd, at)
+    scale = np.linalg.norm(ax) * np.linalg.norm(y)
+    assert abs(float(at.cpu().numpy() @ x) - float(y @ ax)) <= 1e-13 * scale
