@@ -1441,25 +1441,23 @@ __global__ __launch_bounds__(64) void k_q2m_mats(const Pnl *__restrict__ pnl, co
 // every load is one coalesced run over several columns; the passes are
 // unrolled so that several loads per thread are in flight.  The rows' partial
 // sums are added in row order at the end.
-// swap: the transposed L2P of the adjoint operator (Q1 x_n, Q0 x).
 template <typename R, int V>
 __global__ __launch_bounds__(256) void k_q2m(const R *__restrict__ Q0, const R *__restrict__ Q1,
                                              const int *__restrict__ leafStart, const int *__restrict__ leafCount,
                                              const double *__restrict__ x, R *__restrict__ mom, int n, int nm,
-                                             int nmMax, int swap) {
+                                             int nmMax) {
   typedef R VT __attribute__((ext_vector_type(V)));
   R *sm = reinterpret_cast<R *>(dynLds);   // [2][256 V] partial sums: (row, slot)
   const int L = blockIdx.x, t = threadIdx.x, G = nm / V;
   const int rows = max(1, 256 / G), g = t % G, r = t / G;
   const int s = leafStart[L], c = leafCount[L];
-  const int oP = swap ? n : 0, oN = swap ? 0 : n;
   VT m0 = (R)0, m1 = (R)0;
   if (r < rows) {
 #pragma unroll 4
     for (int j = r; j < c; j += rows) {
       const long long col = (long long)(s + j) * nm + g * V;
-      m0 += *reinterpret_cast<const VT *>(Q1 + col) * (R)x[s + j + oP];
-      m1 += *reinterpret_cast<const VT *>(Q0 + col) * (R)x[s + j + oN];
+      m0 += *reinterpret_cast<const VT *>(Q1 + col) * (R)x[s + j];
+      m1 += *reinterpret_cast<const VT *>(Q0 + col) * (R)x[s + j + n];
     }
     for (int v = 0; v < V; v++) {
       sm[r * nm + g * V + v] = m0[v];
@@ -1475,6 +1473,83 @@ __global__ __launch_bounds__(256) void k_q2m(const R *__restrict__ Q0, const R *
     }
     mom[(long long)L * 2 * nmMax + k] = v0;
     mom[(long long)L * 2 * nmMax + nmMax + k] = v1;
+  }
+}
+
+// The FP64 leaf moments.  A panel's noment column is its moment column shifted,
+// N[b] = sum_d n_d M[b - e_d] (moments.c:115-133), so the pass reads the moment
+// matrix alone and keeps four sums per slot,
+//   S[a] = sum_j x_j' M_j[a]  (mom_dpdn),  R_d[a] = sum_j n_jd x_j M_j[a],
+// and forms mom_pot[b] = sum_d R_d[b - e_d] once per leaf.  HBM bounds it: half
+// the bytes of reading both matrices (k_q2m), which is why it is the FP64 form;
+// the FP32 operator keeps the matrices' own rounding.  One block per leaf, four
+// waves over its panels, lanes over slots (V consecutive ones, NL strides of 64
+// lanes), four panels' loads in flight per wave, the panels' weights staged in
+// LDS; the waves' sums are added in wave order.  317k panels, order 6:
+// 90 -> 61 us; 655k panels, order 8: 470 -> 306 us.
+// swap: the transposed L2P of the adjoint operator (the densities exchanged).
+template <int V, int NL>
+__global__ __launch_bounds__(256) void k_q2m64(const double *__restrict__ Q0, const double4 *__restrict__ PN,
+                                               const int *__restrict__ leafStart, const int *__restrict__ leafCount,
+                                               const double *__restrict__ x, double *__restrict__ mom, int n, int nm,
+                                               int nmMax, int swap, DevTabs T) {
+  typedef double VT __attribute__((ext_vector_type(V)));
+  double *red = reinterpret_cast<double *>(dynLds);   // [wave][S, R_x, R_y, R_z][slot]
+  const int L = blockIdx.x, t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int s = leafStart[L], c = leafCount[L];
+  const double *xN = x + s + (swap ? n : 0), *xM = x + s + (swap ? 0 : n);
+  __shared__ double4 wt[256];   // a panel's weights (x', n x)
+  VT a[4][NL];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int q = 0; q < NL; q++) a[k][q] = (VT)0.0;
+  for (int c0 = 0; c0 < c; c0 += 256) {
+    const int cn = min(256, c - c0);
+    __syncthreads();
+    if (t < cn) {
+      const double4 nr = PN[s + c0 + t];
+      const double v = xN[c0 + t];
+      wt[t] = make_double4(xM[c0 + t], nr.x * v, nr.y * v, nr.z * v);
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int j = w; j < cn; j += 4) {
+      const double *col = Q0 + (long long)(s + c0 + j) * nm;
+      const double4 f = wt[j];
+#pragma unroll
+      for (int q = 0; q < NL; q++) {
+        const int i = (lane + 64 * q) * V;
+        if (i < nm) {
+          const VT m = *reinterpret_cast<const VT *>(col + i);
+          a[0][q] += m * f.x;
+          a[1][q] += m * f.y;
+          a[2][q] += m * f.z;
+          a[3][q] += m * f.w;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int q = 0; q < NL; q++) {
+      const int i = (lane + 64 * q) * V;
+      if (i < nm)
+        for (int v = 0; v < V; v++) red[(w * 4 + k) * nm + i + v] = a[k][q][v];
+    }
+  __syncthreads();
+  auto sum = [&](int k, int i) {
+    return ((red[k * nm + i] + red[(4 + k) * nm + i]) + red[(8 + k) * nm + i]) + red[(12 + k) * nm + i];
+  };
+  for (int b = t; b < nm; b += 256) {
+    const int4 m = T.mi[b], e = T.ep[b];   // the moment table: ep = (b - e1, b - e2, b - e3)
+    double v = 0.0;
+    if (m.x & 0xff) v += sum(1, e.x);
+    if ((m.x >> 8) & 0xff) v += sum(2, e.y);
+    if ((m.x >> 16) & 0xff) v += sum(3, e.z);
+    mom[(long long)L * 2 * nmMax + b] = v;
+    mom[(long long)L * 2 * nmMax + nmMax + b] = sum(0, b);
   }
 }
 
@@ -1954,10 +2029,8 @@ __global__ __launch_bounds__(512) void k_l2l(int levStart, const int *__restrict
 // nm / V threads read the columns V slots at a time in coalesced runs; each
 // thread leaves its V-slot partial dot product in LDS and one thread per panel
 // adds the row's partials in slot order.
-// TR: the transposed Q2M of the adjoint operator, from the adjoint moments
-// (M_pot | M_dpdn): far[p] = Q2M1^T M_pot, far[p+n] = Q2M0^T M_dpdn
 #define L2P_CH 32
-template <typename R, int V, bool TR = false>
+template <typename R, int V>
 __global__ __launch_bounds__(256) void k_l2p(const R *__restrict__ Q0, const R *__restrict__ Q1,
                                              const int *__restrict__ leafStart, const int *__restrict__ leafCount,
                                              const R *__restrict__ lec, R *__restrict__ far, int n, int nm,
@@ -1967,18 +2040,10 @@ __global__ __launch_bounds__(256) void k_l2p(const R *__restrict__ Q0, const R *
   R *L12 = sm, *L34 = sm + nm, *P0 = sm + 2 * nm;   // P0/P1: [L2P_CH][G] partial dot products
   const int L = blockIdx.x, t = threadIdx.x, G = nm / V;
   R *P1 = P0 + L2P_CH * G;
-  if constexpr (TR) {
-    const R *l = lec + (long long)L * 2 * nmMax;
-    for (int a = t; a < nm; a += blockDim.x) {
-      L12[a] = l[nmMax + a];
-      L34[a] = l[a];
-    }
-  } else {
-    const R *l = lec + (long long)L * 4 * nmMax;
-    for (int a = t; a < nm; a += blockDim.x) {
-      L12[a] = l[a] + l[nmMax + a];
-      L34[a] = l[2 * nmMax + a] + l[3 * nmMax + a];
-    }
+  const R *l = lec + (long long)L * 4 * nmMax;
+  for (int a = t; a < nm; a += blockDim.x) {
+    L12[a] = l[a] + l[nmMax + a];
+    L34[a] = l[2 * nmMax + a] + l[3 * nmMax + a];
   }
   __syncthreads();
   const int rows = max(1, 256 / G), g = t % G, r = t / G, s = leafStart[L], c = leafCount[L];
@@ -2011,8 +2076,8 @@ __global__ __launch_bounds__(256) void k_l2p(const R *__restrict__ Q0, const R *
         t0 += P0[jj * G + k];
         t1 += P1[jj * G + k];
       }
-      far[s + j0 + jj + (TR ? n : 0)] = t0;
-      far[s + j0 + jj + (TR ? 0 : n)] = t1;
+      far[s + j0 + jj] = t0;
+      far[s + j0 + jj + n] = t1;
     }
     __syncthreads();
   }
@@ -2156,6 +2221,144 @@ __global__ __launch_bounds__(256) void k_l2lp(const R *__restrict__ Q0, const R 
       far[s0 + j0 + jj + n] = t1;
     }
     __syncthreads();
+  }
+}
+
+// The FP64 downward pass of one leaf: L2L down its ancestry and L2P as k_l2lp,
+// on the two sums the panels need (u = l1 + l2 against the moments, v = l3 + l4
+// against the noments; translation is linear, so they are formed before it) and
+// with the moment matrix alone: N[b] = sum_d n_d M[b - e_d] gives
+//   far[p] = sum_a M[a] u[a],  far[p + n] = sum_a M[a] (n . g[a]),  g_d[a] = v[a + e_d].
+// A wave takes four panels at a time, lanes over slots with u and g of their
+// slots in registers; the eight sums are reduced together, halving the values
+// with the lanes (10 exchanges instead of 48).  HBM bounds it (one column per
+// panel).  317k panels, order 6: 122 -> 119 us; 655k panels, order 8 (which had
+// no fused form: its partial sums did not fit in LDS): 1,715 -> 318 us.
+// TR: the transposed M2M and Q2M of the adjoint operator, from the adjoint
+// moments (M_pot | M_dpdn): far[p] = N . M_pot, far[p + n] = M . M_dpdn.
+template <int V, int NL, bool TR>
+__global__ __launch_bounds__(256) void k_l2lp64(const double *__restrict__ Q0, const double4 *__restrict__ PN,
+                                                const int *__restrict__ leafStart, const int *__restrict__ leafCount,
+                                                const int *__restrict__ anc, LevOrd O,
+                                                const double *__restrict__ cubeX, const double *__restrict__ lec,
+                                                double *__restrict__ far, int n, int nm, int nmMax, int nUp, int nAnc,
+                                                DevTabs T) {
+  typedef double VT __attribute__((ext_vector_type(V)));
+  __shared__ double co[L2LP_MAXUP][3][MAXP + 1];   // t_d^k / k! of each step
+  __shared__ double4 wt[256];                      // the panels' normals
+  const int L = blockIdx.x, t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int s0 = leafStart[L], c = leafCount[L];
+  // chain(nUp) = the leaf, chain(s - 1) = parent of chain(s)
+  auto chain = [&](int s) { return anc[(long long)L * nAnc + nUp - s]; };
+  // (u, v) per slot: two working buffers, then the M2L locals of chain(1..nUp)
+  double2 *cur = reinterpret_cast<double2 *>(dynLds), *nxt = cur + nmMax, *own = nxt + nmMax;
+  const int4 mt = T.mi[min(t, nmMax - 1)];   // a thread owns slot t (nMom(9) = 220)
+  for (int s = 0; s <= nUp; s++)   // every local the block needs, loads all in flight at once
+    if (t < nmMax) {
+      const double *l = lec + (long long)chain(s) * (TR ? 2 : 4) * nmMax;
+      double2 *dst = s == 0 ? cur : own + (s - 1) * nmMax;
+      if constexpr (TR) dst[t] = make_double2(l[nmMax + t], l[t]);
+      else dst[t] = make_double2(l[t] + l[nmMax + t], l[2 * nmMax + t] + l[3 * nmMax + t]);
+    }
+  if (t < 3 * nUp) {
+    const int s = t / 3 + 1, d = t % 3;
+    const double tr = cubeX[3 * chain(s) + d] - cubeX[3 * chain(s - 1) + d];
+    double f = 1.0;
+    for (int k = 0; k <= O.p[s - 1]; k++) {
+      co[s - 1][d][k] = f;
+      f = f * tr / (k + 1);
+    }
+  }
+  const int i1 = mt.x & 0xff, i2 = (mt.x >> 8) & 0xff, i3 = (mt.x >> 16) & 0xff;
+  __syncthreads();
+  for (int s = 1; s <= nUp; s++) {
+    const int pin = O.p[s - 1], nIn = NMOM(pin), nOut = NMOM(O.p[s]);
+    for (int d = 2; d >= 0; d--) {   // z, y, x
+      const double *cd = co[s - 1][d];
+      if (t < (d == 0 ? nOut : nIn)) {
+        const int kmax = pin - deg_of(mt);
+        double2 u = make_double2(0.0, 0.0);
+        for (int k = 0; k <= kmax; k++) {
+          const double2 v = cur[idx3(i1 + (d == 0 ? k : 0), i2 + (d == 1 ? k : 0), i3 + (d == 2 ? k : 0))];
+          u.x += cd[k] * v.x;
+          u.y += cd[k] * v.y;
+        }
+        if (d == 0) {   // the kid's own M2L locals
+          const double2 o = own[(s - 1) * nmMax + t];
+          u.x += o.x;
+          u.y += o.y;
+        }
+        nxt[t] = u;
+      }
+      __syncthreads();
+      double2 *sw = cur;
+      cur = nxt;
+      nxt = sw;
+    }
+  }
+  const int nG = O.p[nUp] > 0 ? NMOM(O.p[nUp] - 1) : 0;
+  VT u[NL], gx[NL], gy[NL], gz[NL];
+#pragma unroll
+  for (int q = 0; q < NL; q++)
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      const int a = (lane + 64 * q) * V + v;
+      const int4 e = a < nG ? T.ep[a] : make_int4(0, 0, 0, 0);   // a + e1, a + e2, a + e3
+      u[q][v] = a < nm ? cur[a].x : 0.0;
+      gx[q][v] = a < nG ? cur[e.x].y : 0.0;
+      gy[q][v] = a < nG ? cur[e.y].y : 0.0;
+      gz[q][v] = a < nG ? cur[e.z].y : 0.0;
+    }
+  for (int c0 = 0; c0 < c; c0 += 256) {
+    const int cn = min(256, c - c0);
+    __syncthreads();
+    if (t < cn) wt[t] = PN[s0 + c0 + t];
+    __syncthreads();
+    VT m[4][NL];
+    auto fetch = [&](int j0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const double *col = Q0 + (long long)(s0 + c0 + min(j0 + k, cn - 1)) * nm;
+#pragma unroll
+        for (int q = 0; q < NL; q++) {
+          const int i = (lane + 64 * q) * V;
+          m[k][q] = i < nm ? *reinterpret_cast<const VT *>(col + i) : (VT)0.0;
+        }
+      }
+    };
+    if (4 * w < cn) fetch(4 * w);
+    for (int j0 = 4 * w; j0 < cn; j0 += 16) {
+      double v8[8];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const double4 nr = wt[min(j0 + k, cn - 1)];
+        double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+        for (int q = 0; q < NL; q++) {
+          const VT g = nr.x * gx[q] + nr.y * gy[q] + nr.z * gz[q];
+          for (int v = 0; v < V; v++) {
+            t0 += m[k][q][v] * u[q][v];
+            t1 += m[k][q][v] * g[v];
+          }
+        }
+        v8[2 * k] = t0;
+        v8[2 * k + 1] = t1;
+      }
+      if (j0 + 16 < cn) fetch(j0 + 16);   // in flight under the reduction
+#pragma unroll
+      for (int h = 4, o = 32; h > 0; h >>= 1, o >>= 1) {   // a lane keeps the half its bit o selects
+        const bool up = lane & o;
+#pragma unroll
+        for (int k = 0; k < h; k++) {
+          const double keep = up ? v8[k + h] : v8[k], give = up ? v8[k] : v8[k + h];
+          v8[k] = keep + __shfl_xor(give, o, 64);
+        }
+      }
+      double r = v8[0];
+      for (int o = 4; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
+      const int k = lane >> 4, which = (lane >> 3) & 1;
+      if ((lane & 7) == 0 && j0 + k < cn) far[s0 + c0 + j0 + k + (which != (TR ? 1 : 0) ? n : 0)] = r;
+    }
   }
 }
 
@@ -4163,10 +4366,12 @@ struct fbh_ctx {
   long long *specOff = nullptr;
   int *specCol = nullptr;
   long long nSpec = 0;
-  // FP64 nearfield on the fly (q = 1): panel data and the corrections in FP64
+  // FP64 panel data (first quadrature point and area, normal; the far passes read
+  // the normals too) and the nearfield on the fly (q = 1): corrections in FP64
   bool fly64 = false;
   double4 *fly64PA = nullptr, *fly64PN = nullptr, *specVal64 = nullptr, *specValT64 = nullptr;
   NearK nearK[2] = {};          // its constants: the operator's rows and the transposed ones
+  int *leafAnc = nullptr;       // each leaf and its ancestors, finest first (depth - height + 1 entries)
   NearTile *nearDesc = nullptr; // its tiles in launch order
   double *nearTab = nullptr;    // e^{-kappa r} at the steps of NearK
   double *ro = nullptr, *dx = nullptr;   // refinement residual and correction
@@ -4888,6 +5093,18 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
     FAIL();
   }
 
+  {   // each leaf's ancestry, and the panels' points and normals
+    const int na = depth - height + 1;
+    std::vector<int> anc((size_t)nLeaf * na);
+    for (int l = 0; l < nLeaf; l++)
+      for (int s = 0, cb = l; s < na; s++, cb = s < na ? parent[cb] : cb) anc[(size_t)l * na + s] = cb;
+    if (!(c->leafAnc = dupload(c, anc.data(), anc.size())) || !(c->fly64PA = dalloc<double4>(c, n)) ||
+        !(c->fly64PN = dalloc<double4>(c, n)))
+      FAIL();
+    hipLaunchKernelGGL(k_fly64_panels, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->pnl, n, c->Q.t[0],
+                       c->fly64PA, c->fly64PN);
+    if (hipGetLastError() != hipSuccess) { setErr("k_fly64_panels launch failed"); FAIL(); }
+  }
   // leaf Q2M/L2P matrices on the device
   {
     size_t lds = 5 * (size_t)c->nmLeaf * sizeof(double);
@@ -5123,37 +5340,67 @@ static int vecWidth(int nm) {
   return nm % v == 0 ? v : nm % 2 == 0 ? 2 : 1;
 }
 template <typename R>
-static void launchQ2M(const fbh_ctx *c, const R *Q0, const R *Q1, const double *x, R *mom, int swap, hipStream_t st) {
+static void launchQ2M(const fbh_ctx *c, const R *Q0, const R *Q1, const double *x, R *mom, hipStream_t st) {
   const int V = vecWidth<R>(c->nmLeaf);
   const size_t lds = 512 * (size_t)V * sizeof(R);
-  if (V == 4)
-    hipLaunchKernelGGL((k_q2m<R, 4>), dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, x, mom,
-                       c->n, c->nmLeaf, c->nmMax, swap);
-  else if (V == 2)
-    hipLaunchKernelGGL((k_q2m<R, 2>), dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, x, mom,
-                       c->n, c->nmLeaf, c->nmMax, swap);
-  else
-    hipLaunchKernelGGL((k_q2m<R, 1>), dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, x, mom,
-                       c->n, c->nmLeaf, c->nmMax, swap);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, x, mom, c->n,
+                       c->nmLeaf, c->nmMax);
+  };
+  if (V == 4) launch(k_q2m<R, 4>);
+  else if (V == 2) launch(k_q2m<R, 2>);
+  else launch(k_q2m<R, 1>);
 }
-template <typename R, bool TR = false>
+template <typename R>
 static void launchL2P(const fbh_ctx *c, const R *Q0, const R *Q1, const R *lec, R *far, hipStream_t st) {
   const int V = vecWidth<R>(c->nmLeaf), G = c->nmLeaf / V;
   const size_t lds = (2 * (size_t)c->nmLeaf + 2 * (size_t)L2P_CH * G) * sizeof(R);
-  if (V == 4)
-    hipLaunchKernelGGL((k_l2p<R, 4, TR>), dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, lec,
-                       far, c->n, c->nmLeaf, c->nmMax);
-  else if (V == 2)
-    hipLaunchKernelGGL((k_l2p<R, 2, TR>), dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, lec,
-                       far, c->n, c->nmLeaf, c->nmMax);
-  else
-    hipLaunchKernelGGL((k_l2p<R, 1, TR>), dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, lec,
-                       far, c->n, c->nmLeaf, c->nmMax);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(c->nLeaf), dim3(256), lds, st, Q0, Q1, c->leafStart, c->leafCount, lec, far, c->n,
+                       c->nmLeaf, c->nmMax);
+  };
+  if (V == 4) launch(k_l2p<R, 4>);
+  else if (V == 2) launch(k_l2p<R, 2>);
+  else launch(k_l2p<R, 1>);
+}
+
+// The FP64 passes over the moment matrix: a wave's lanes cover a column of nMom
+// slots, two slots a lane where the column's length (so every column's start) is
+// even, one where it is odd (orders 4 and 8); f(V, NL) with NL strides of 64 lanes.
+template <class F>
+static void withSlots(int nm, F f) {
+  using std::integral_constant;
+  if (nm % 2 == 0) {
+    if (nm <= 128) f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else f(integral_constant<int, 2>{}, integral_constant<int, 2>{});   // order 9: 220
+  } else {
+    if (nm <= 64) f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else f(integral_constant<int, 1>{}, integral_constant<int, 3>{});   // order 8: 165
+  }
+}
+static void q2m64(const fbh_ctx *c, const double *x, double *mom, int swap, hipStream_t st) {
+  withSlots(c->nmLeaf, [&](auto V, auto NL) {
+    hipLaunchKernelGGL((k_q2m64<V.value, NL.value>), dim3(c->nLeaf), dim3(256), 16 * (size_t)c->nmLeaf * sizeof(double),
+                       st, c->Q0, c->fly64PN, c->leafStart, c->leafCount, x, mom, c->n, c->nmLeaf, c->nmMax, swap, c->Tm);
+  });
+}
+// nUp: levels translated down before the L2P (0: from the leaves' own locals)
+template <bool TR>
+static void l2lp64(const fbh_ctx *c, const double *lec, double *far, int nUp, hipStream_t st) {
+  LevOrd O{};
+  for (int s = 0; s <= nUp; s++) O.p[s] = c->ordMom[c->depth - nUp + s];
+  const size_t lds = (size_t)(nUp + 2) * c->nmMax * sizeof(double2);
+  withSlots(c->nmLeaf, [&](auto V, auto NL) {
+    hipLaunchKernelGGL((k_l2lp64<V.value, NL.value, TR>), dim3(c->nLeaf), dim3(256), lds, st, c->Q0, c->fly64PN,
+                       c->leafStart, c->leafCount, c->leafAnc, O, c->cubeX, lec, far, c->n, c->nmLeaf, c->nmMax, nUp,
+                       c->depth - c->height + 1, c->T);
+  });
 }
 
 template <typename R>
 static void q2mPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_t st) {
-  launchQ2M<R>(c, B.Q0, B.Q1, x, B.mom, 0, st);
+  if constexpr (std::is_same<R, double>::value) q2m64(c, x, B.mom, 0, st);
+  else launchQ2M<R>(c, B.Q0, B.Q1, x, B.mom, st);
 }
 
 template <typename R>   // children at lev + 1 into parents at lev
@@ -5176,13 +5423,15 @@ static void l2lPass(fbh_ctx *c, const OpBufs<R> &B, int lev, hipStream_t st) {
 
 template <typename R>
 static void l2pPass(fbh_ctx *c, const OpBufs<R> &B, hipStream_t st) {
-  launchL2P<R>(c, B.Q0, B.Q1, B.lec, B.far, st);
+  if constexpr (std::is_same<R, double>::value) l2lp64<false>(c, B.lec, B.far, 0, st);
+  else launchL2P<R>(c, B.Q0, B.Q1, B.lec, B.far, st);
 }
 
 // L2L (every level) and L2P in one launch; the locals in B.lec stay the M2L ones.
 // False (nothing launched) when the block's tables do not fit in LDS.
 template <typename R>
 static size_t l2lpLds(const fbh_ctx *c) {
+  if (std::is_same<R, double>::value) return (size_t)(c->depth - c->height + 2) * c->nmMax * sizeof(double2);
   const int V = vecWidth<R>(c->nmLeaf), G = c->nmLeaf / V;
   return std::max(4 * (size_t)(c->depth - c->height + 2) * c->nmMax * sizeof(R),
                   2 * (size_t)L2P_CH * G * sizeof(R));
@@ -5194,29 +5443,37 @@ static bool l2lpFits(const fbh_ctx *c) {
 template <typename R>
 static bool l2lpPass(fbh_ctx *c, const OpBufs<R> &B, hipStream_t st) {
   if (!l2lpFits<R>(c)) return false;
-  const int V = vecWidth<R>(c->nmLeaf), nmx = c->nmMax, nUp = c->depth - c->height;
-  const size_t lds = l2lpLds<R>(c);
-  LevOrd O{};
-  for (int s = 0; s <= nUp; s++) O.p[s] = c->ordMom[c->height + s];
-  if (V == 4)
-    hipLaunchKernelGGL((k_l2lp<R, 4>), dim3(c->nLeaf), dim3(256), lds, st, B.Q0, B.Q1, c->leafStart, c->leafCount,
-                       c->parent, O, c->cubeX, B.lec, B.far, c->n, c->nmLeaf, nmx, nUp, c->T);
-  else if (V == 2)
-    hipLaunchKernelGGL((k_l2lp<R, 2>), dim3(c->nLeaf), dim3(256), lds, st, B.Q0, B.Q1, c->leafStart, c->leafCount,
-                       c->parent, O, c->cubeX, B.lec, B.far, c->n, c->nmLeaf, nmx, nUp, c->T);
-  else
-    hipLaunchKernelGGL((k_l2lp<R, 1>), dim3(c->nLeaf), dim3(256), lds, st, B.Q0, B.Q1, c->leafStart, c->leafCount,
-                       c->parent, O, c->cubeX, B.lec, B.far, c->n, c->nmLeaf, nmx, nUp, c->T);
+  if constexpr (std::is_same<R, double>::value) {
+    l2lp64<false>(c, B.lec, B.far, c->depth - c->height, st);
+  } else {
+    const int V = vecWidth<R>(c->nmLeaf), nmx = c->nmMax, nUp = c->depth - c->height;
+    const size_t lds = l2lpLds<R>(c);
+    LevOrd O{};
+    for (int s = 0; s <= nUp; s++) O.p[s] = c->ordMom[c->height + s];
+    if (V == 4)
+      hipLaunchKernelGGL((k_l2lp<R, 4>), dim3(c->nLeaf), dim3(256), lds, st, B.Q0, B.Q1, c->leafStart, c->leafCount,
+                         c->parent, O, c->cubeX, B.lec, B.far, c->n, c->nmLeaf, nmx, nUp, c->T);
+    else if (V == 2)
+      hipLaunchKernelGGL((k_l2lp<R, 2>), dim3(c->nLeaf), dim3(256), lds, st, B.Q0, B.Q1, c->leafStart, c->leafCount,
+                         c->parent, O, c->cubeX, B.lec, B.far, c->n, c->nmLeaf, nmx, nUp, c->T);
+    else
+      hipLaunchKernelGGL((k_l2lp<R, 1>), dim3(c->nLeaf), dim3(256), lds, st, B.Q0, B.Q1, c->leafStart, c->leafCount,
+                         c->parent, O, c->cubeX, B.lec, B.far, c->n, c->nmLeaf, nmx, nUp, c->T);
+  }
   return true;
 }
 
-// M2M of one level by axis-wise translation (k_m2m_ax); false when its LDS does not fit
+// M2M of one level by axis-wise translation (k_m2m_ax), a wave per child where
+// their buffers fit in LDS, else four waves (FP64 at orders 8 and 9);
+// false when they do not fit either
 template <typename R>
 static bool m2mAxPass(fbh_ctx *c, const OpBufs<R> &B, int lev, hipStream_t st) {
-  const size_t lds = (24 * (size_t)c->nmMax * 2 + 8 * 3 * (MAXP + 1)) * sizeof(R);
+  auto need = [&](int nw) { return ((8 + 2 * nw) * (size_t)c->nmMax * 2 + nw * 3 * (MAXP + 1)) * sizeof(R); };
+  const int nw = need(8) <= (size_t)c->ldsMax ? 8 : 4;
+  const size_t lds = need(nw);
   if (lds > (size_t)c->ldsMax) return false;
   if (c->levCount[lev] > 0)
-    hipLaunchKernelGGL(k_m2m_ax<R>, dim3(c->levCount[lev]), dim3(512), lds, st, c->levStart[lev], c->ordMom[lev],
+    hipLaunchKernelGGL(k_m2m_ax<R>, dim3(c->levCount[lev]), dim3(64 * nw), lds, st, c->levStart[lev], c->ordMom[lev],
                        NMOM(c->ordMom[lev + 1]), c->kidStart, c->nKids, c->cubeX, B.mom, c->nmMax, c->T);
   return true;
 }
@@ -5353,10 +5610,11 @@ static int ensureAdjoint(fbh_ctx *c) {
 
 // the transposed far chain from y into c->far (adjL: adjoint locals, adjM: adjoint moments)
 static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
-  launchQ2M<double>(c, c->Q0, c->Q1, y, c->adjL, 1, st);
+  q2m64(c, y, c->adjL, 1, st);
   OpBufs<double> B = bufs64(c);
   B.mom = c->adjL;
-  for (int lev = c->depth - 1; lev >= c->height; lev--) m2mPass(c, B, lev, st);
+  for (int lev = c->depth - 1; lev >= c->height; lev--)
+    if (!m2mAxPass(c, B, lev, st)) m2mPass(c, B, lev, st);
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(c->nCube), dim3(64 * c->m2lWaves), c->m2lLds, st, c->m2lOff, c->m2lSrc,
                        c->cubeLevelD, c->ordM2LD, c->ordMomD, (const double *)c->m2lG, (const double *)c->adjL,
@@ -5366,6 +5624,10 @@ static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
   } else if (c->m2lMaxT == 16) launch(k_m2l_cached<double, 16, true>);
   else if (c->m2lMaxT == 32) launch(k_m2l_cached<double, 32, true>);
   else launch(k_m2l_cached<double, 0, true>);
+  if (l2lpFits<double>(c)) {
+    l2lp64<true>(c, c->adjM, c->far, c->depth - c->height, st);
+    return;
+  }
   for (int lev = c->height; lev < c->depth; lev++) {
     const int nIn = NMOM(c->ordMom[lev]), nOut = NMOM(c->ordMom[lev + 1]);
     if (c->levCount[lev + 1] <= 0) continue;
@@ -5374,7 +5636,7 @@ static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
                        c->levStart[lev + 1], c->parent, c->cubeLevelD, c->ordMomD, c->cubeX, c->adjM, c->nmMax,
                        c->T);
   }
-  launchL2P<double, true>(c, c->Q0, c->Q1, c->adjM, c->far, st);
+  l2lp64<true>(c, c->adjM, c->far, 0, st);
 }
 
 // y = alpha*(D - K)^T x + beta*y
@@ -5458,11 +5720,8 @@ static int enableFly64(fbh_ctx *c, double rMax) {
     o.f1 = sg * e / 3.0;
     o.f2 = sg * (e - 1.0) / 3.0;
   }
-  if (!(c->fly64PA = dalloc<double4>(c, n)) || !(c->fly64PN = dalloc<double4>(c, n)) || !ensureSpec(c) ||
-      !(c->specVal64 = dalloc<double4>(c, (size_t)c->nSpec)))
+  if (!ensureSpec(c) || !(c->specVal64 = dalloc<double4>(c, (size_t)c->nSpec)))
     return 0;
-  hipLaunchKernelGGL(k_fly64_panels, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->pnl, (int)n, c->Q.t[0],
-                     c->fly64PA, c->fly64PN);
   hipLaunchKernelGGL(k_exp2_tab, dim3(1), dim3(256), 0, c->stream);
   hipLaunchKernelGGL(k_spec_vals<false>, dim3(n), dim3(64), 0, c->stream, c->pnl, c->specOff, c->specCol,
                      (float4 *)nullptr, c->specVal64, c->kappa, c->eps, c->Q, c->qorder);
@@ -6510,10 +6769,12 @@ static int kappaOperatorTerms(fbh_ctx *c, const double *sgm_dev, const double *l
   if (ok) {   // far part: moments of u, adjoint locals of lam, the kappa-differentiated M2L between them
     OpBufs<double> B = bufs64(c);
     q2mPass(c, B, sgm_dev, c->stream);
-    for (int lev = c->depth - 1; lev >= c->height; lev--) m2mPass(c, B, lev, c->stream);
-    launchQ2M<double>(c, c->Q0, c->Q1, lam_dev, c->adjL, 1, c->stream);
+    for (int lev = c->depth - 1; lev >= c->height; lev--)
+      if (!m2mAxPass(c, B, lev, c->stream)) m2mPass(c, B, lev, c->stream);
+    q2m64(c, lam_dev, c->adjL, 1, c->stream);
     B.mom = c->adjL;
-    for (int lev = c->depth - 1; lev >= c->height; lev--) m2mPass(c, B, lev, c->stream);
+    for (int lev = c->depth - 1; lev >= c->height; lev--)
+      if (!m2mAxPass(c, B, lev, c->stream)) m2mPass(c, B, lev, c->stream);
     if (c->gridK && c->m2lG && !c->m2lGdk) {   // (dGk/dkappa, Gk) per pair, cached as the M2L tensors are
       if (!(c->m2lGdk = dalloc<double>(c, (size_t)c->nM2L * 2 * c->nmMax))) return 0;
       hipLaunchKernelGGL(k_m2l_derivs, dim3((unsigned)c->nM2L), dim3(64),

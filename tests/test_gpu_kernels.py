@@ -44,3 +44,22 @@ def test_near_exponential_table(fa, tmp_path_factory, kappa, depth):
     op.matvec_t_dev(yd, at)
     scale = np.linalg.norm(ax) * np.linalg.norm(y)
     assert abs(float(at.cpu().numpy() @ x) - float(y @ ax)) <= 1e-13 * scale
+
+
+@pytest.mark.parametrize("order,depth,mac", [(1, 2, 0.8), (3, 3, 0.8), (4, 2, 0.8), (7, 2, 0.8), (8, 3, 0.7), (9, 2, 0.8)])
+def test_far_chain_orders(fa, tmp_path_factory, order, depth, mac):
+    """Q2M and L2P from the moment matrix alone, for every split of a column over a wave's
+    lanes (one or two slots, one to three strides), forward and transposed."""
+    import torch
+    mesh = molecule(fa, tmp_path_factory, "globule", 3, 8, *GLOBULE)
+    tree = fa.Tree(mesh, depth, order=order, sep=mac)
+    op = fa.Operator(tree, 0.1257, 1.0, 80.0, 1)
+    x, y = np.random.default_rng(2).uniform(-1, 1, (2, 2 * tree.n))
+    ora = O.Oracle(tree.oracle_layout(0.1257, 1.0, 80.0, 1))
+    ax = op.matvec(x)
+    assert rel(ax, ora.matvec(x)) <= 1e-13
+    assert rel(op.far_apply(x), ora.apply(x, parts=1)) <= 1e-13   # the stage form
+    yd = torch.tensor(y, device="cuda")
+    at = torch.empty_like(yd)
+    op.matvec_t_dev(yd, at)
+    assert abs(float(at.cpu().numpy() @ x) - float(y @ ax)) <= 1e-13 * np.linalg.norm(ax) * np.linalg.norm(y)
