@@ -562,6 +562,41 @@ __device__ __forceinline__ T waveSumT(T v) {
   return v;
 }
 
+// lane exchanges without LDS: the upper half (32) or the odd rows of 16 lanes (16)
+// of a trade places with the other half of b; a + b afterwards adds the halves of
+// a in the lanes that kept it and of b in the others
+template <int O>
+__device__ __forceinline__ double swapAdd(double a, double b) {
+  const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
+  if constexpr (O == 32) {
+    const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+  }
+}
+template <int CTRL>
+__device__ __forceinline__ double dppMove(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false));
+}
+// the wave sums of eight values: lane l returns the sum of v[l >> 3]
+__device__ __forceinline__ double waveSum8(double (&v)[8], int lane) {
+#pragma unroll
+  for (int k = 0; k < 4; k++) v[k] = swapAdd<32>(v[k], v[k + 4]);
+#pragma unroll
+  for (int k = 0; k < 2; k++) v[k] = swapAdd<16>(v[k], v[k + 2]);
+  const bool up = lane & 8;
+  double r = (up ? v[1] : v[0]) + dppMove<0x128>(up ? v[0] : v[1]);   // row_ror:8
+  r += dppMove<0xB1>(r);    // quad_perm [1,0,3,2]
+  r += dppMove<0x4E>(r);    // quad_perm [2,3,0,1]
+  r += dppMove<0x141>(r);   // row_half_mirror
+  return r;
+}
+
 template <typename R> struct Vec4;
 template <> struct Vec4<double> { typedef double4 type; };
 template <> struct Vec4<float> { typedef float4 type; };
@@ -1856,10 +1891,8 @@ __global__ __launch_bounds__(256) void k_m2l_cached(const int *__restrict__ m2lO
 // registers into one [run][lane] table in wave order and one thread per alpha
 // sums the cells that hold it (a fixed list), then combines the four sums
 //   t1 = sum c1 a0, t2 = sum c1 ak, t3 = sum c2 a0, t4 = sum c2 ak
-// into the locals (TR: into the adjoint moments), as k_m2l_cached does per item.
-// DK: G holds (dGk/dkappa, Gk) and the output is the raw pair (t1, t3), the
-// moments against dGk/dkappa (the kappa derivative of the far operator).
-template <typename R, int K, int L, bool TR = false, bool DK = false>
+// into the locals, as k_m2l_cached does per item.  The FP32 operator's M2L.
+template <typename R, int K, int L>
 __global__ __launch_bounds__(256) void k_m2l_grid(const int *__restrict__ m2lOff, const int *__restrict__ m2lSrc,
                                                   const int *__restrict__ cubeLevel, const int *__restrict__ ordM2L,
                                                   const int *__restrict__ ordMom, const R *__restrict__ G,
@@ -1954,11 +1987,8 @@ __global__ __launch_bounds__(256) void k_m2l_grid(const int *__restrict__ m2lOff
   }
   const int nmc = NMOM(ordMom[cubeLevel[c]]);
   const int *rs = redStart + gridOff[2 * p + 1];
-  constexpr int NO = TR || DK ? 2 : 4;
   for (int a = tid; a < nmMax; a += blockDim.x) {
-    R v[NO];
-#pragma unroll
-    for (int k = 0; k < NO; k++) v[k] = 0;
+    R v[4] = {0, 0, 0, 0};
     if (a < nm && a < nmc) {
       R t1 = 0, t2 = 0, t3 = 0, t4 = 0;
       for (int i = rs[a]; i < rs[a + 1]; i++) {
@@ -1968,6 +1998,182 @@ __global__ __launch_bounds__(256) void k_m2l_grid(const int *__restrict__ m2lOff
         t3 += q[2];
         t4 += q[3];
       }
+      v[0] = t3 - t4;
+      v[1] = eps * t2 - t1;
+      v[2] = t3 - t4 / eps;
+      v[3] = t2 - t1;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) lec[((long long)c * 4 + k) * nmMax + a] = v[k];
+  }
+}
+
+// The FP64 M2L from cached tensors (src/fmm.c:774-787, src/expan.c:258-290,
+// 471-494), organised by the tensor slot: l[alpha] = sum_beta c[beta] v[alpha +
+// beta] is run with one slot gamma = alpha + beta per lane for the whole
+// interaction list, so a lane reads a pair's D G0[gamma], D Gk[gamma] from LDS
+// once and then one 16-byte (c1, c2) moment slot per four FMAs; k_m2l_grid, whose
+// lanes keep alpha instead, reads two slots per four FMAs, and LDS reads bound it.
+// The host (planGamma) deals the products beta <= gamma into cells of L betas of
+// one gamma, one cell per lane of W waves; step l of lane has a fixed alpha =
+// gamma - beta, so its four sums
+//   t1 = sum c1 a0, t2 = sum c1 ak, t3 = sum c2 a0, t4 = sum c2 ak
+// stay in registers.  GR groups of W waves take every GR-th batch of NB pairs,
+// staged by all of a group's threads (coalesced, two batches ahead in registers,
+// two LDS buffers, one barrier per batch).  After the list the lanes' sums pass
+// through LDS, NC of the four at a time, and are added per alpha in a fixed order
+// (segments of GAMMA_SEG entries, one thread and one 16-byte load each, then the
+// segments of an alpha).
+// 81,920 panels, order 6: 58 -> 44 us; 317k: 181 -> 140; 655k, order 8: 2,400 ->
+// 1,660 (with the tensors gathered straight into registers instead: 58, 242 and
+// 3,565 us, bound by the gathers' address rate).
+// TR: into the adjoint moments.  DK: G holds (dGk/dkappa, Gk) and the output is
+// the raw pair (t1, t3), the moments against dGk/dkappa.
+#define GAMMA_SEG 8
+struct GammaPlan {   // device arrays of one order
+  const int *gamma;              // [cells]
+  const unsigned short *beta;    // [L][cells], the zero slot where a cell is short
+  const unsigned short *ent;     // [nSeg][GAMMA_SEG]: step * cells + cell, padded with the zero entry L * cells
+  const int *alphaSeg;           // [nm + 1] ranges of segments
+  int nSeg;
+};
+struct GammaPlans {
+  GammaPlan p[9];
+};
+struct GammaCube {   // a destination cube, in launch order
+  int cube, b0, b1, p, nOut, pad[3];
+};
+template <int PM, int L, int W, int NB, int NC, bool TR, bool DK>
+__global__ __launch_bounds__(512, 4) void k_m2l_gamma(const GammaCube *__restrict__ cubes, const int *__restrict__ m2lSrc,
+                                                   const double *__restrict__ G, const double *__restrict__ mom,
+                                                   double *__restrict__ lec, int nmMax, double eps, DevTabs T,
+                                                   GammaPlans plans) {
+  constexpr int CELLS = 64 * W, slotZ = NMOM(PM), ncc = slotZ + 1, NK = (NB * slotZ + CELLS - 1) / CELLS;
+  const GammaCube C = cubes[blockIdx.x];
+  const int tid = threadIdx.x, GR = blockDim.x / CELLS, grp = __builtin_amdgcn_readfirstlane(tid / CELLS),
+            cell = tid % CELLS;
+  const int c = C.cube, nm = NMOM(C.p), b0 = C.b0, b1 = C.b1;
+  const GammaPlan P = plans.p[C.p];
+  // [buffer][pair][moments, tensors][ncc]
+  double2 *cc = reinterpret_cast<double2 *>(dynLds) + (size_t)grp * 4 * NB * ncc;
+  if (cell < 4 * NB) cc[cell * ncc + slotZ] = make_double2(0.0, 0.0);
+  const int nt = (b1 - b0 + NB * GR - 1) / (NB * GR);
+  auto start = [&](int t) { return b0 + (t * GR + grp) * NB; };
+  int sq[NK], sl[NK], src[NK];   // the thread's staged slots: pair of the batch, slot
+  double sg[NK], ma[NK], mb[NK], ga[NK], gb[NK];
+#pragma unroll
+  for (int q = 0; q < NK; q++) {
+    const int i = cell + q * CELLS;
+    sq[q] = i / nm;
+    sl[q] = i - sq[q] * nm;
+  }
+  auto valid = [&](int t, int q) { return sq[q] < NB && start(t) + sq[q] < b1; };
+  auto fetchSrc = [&](int t) {
+#pragma unroll
+    for (int q = 0; q < NK; q++)
+      if (valid(t, q)) src[q] = m2lSrc[start(t) + sq[q]];
+  };
+  auto fetch = [&](int t) {
+#pragma unroll
+    for (int q = 0; q < NK; q++)
+      if (valid(t, q)) {
+        const double *g = G + (long long)(start(t) + sq[q]) * 2 * nmMax + sl[q];
+        const double *m = mom + (long long)src[q] * 2 * nmMax + sl[q];
+        ga[q] = g[0];
+        gb[q] = g[nmMax];
+        ma[q] = m[0];
+        mb[q] = m[nmMax];
+      }
+  };
+  auto store = [&](int t) {
+    double2 *d = cc + (t & 1) * 2 * NB * ncc;
+#pragma unroll
+    for (int q = 0; q < NK; q++)
+      if (valid(t, q)) {
+        d[2 * sq[q] * ncc + sl[q]] = make_double2(sg[q] * ma[q], sg[q] * mb[q]);
+        d[(2 * sq[q] + 1) * ncc + sl[q]] = make_double2(ga[q], gb[q]);
+      }
+  };
+  fetchSrc(0);
+#pragma unroll
+  for (int q = 0; q < NK; q++) sg[q] = T.ep[sl[q]].w;
+  int be[L];   // byte offsets of the lane's moments
+#pragma unroll
+  for (int l = 0; l < L; l++) be[l] = P.beta[l * CELLS + cell] * (int)sizeof(double2);
+  const int be0 = (P.gamma[cell] + ncc) * (int)sizeof(double2);   // and of its tensor slot
+  fetch(0);
+  fetchSrc(1);
+  store(0);
+  fetch(1);
+  fetchSrc(2);
+  double acc[L][4];
+#pragma unroll
+  for (int l = 0; l < L; l++) acc[l][0] = acc[l][1] = acc[l][2] = acc[l][3] = 0.0;
+  for (int t = 0; t < nt; t++) {
+    __syncthreads();   // batch t staged; batch t - 1's buffer free
+    const unsigned char *cb = reinterpret_cast<const unsigned char *>(cc + (t & 1) * 2 * NB * ncc);
+#pragma unroll
+    for (int k = 0; k < NB; k++)
+      if (start(t) + k < b1) {
+        const int o = 2 * k * ncc * (int)sizeof(double2);
+        const double2 g = *reinterpret_cast<const double2 *>(cb + be0 + o);
+#pragma unroll
+        for (int l = 0; l < L; l++) {
+          const double2 m = *reinterpret_cast<const double2 *>(cb + be[l] + o);
+          acc[l][0] += m.x * g.x;
+          acc[l][1] += m.x * g.y;
+          acc[l][2] += m.y * g.x;
+          acc[l][3] += m.y * g.y;
+        }
+      }
+    store(t + 1);
+    fetch(t + 2);
+    fetchSrc(t + 3);
+  }
+  // per alpha: red[step * CELLS + cell][NC] and its zero entry, segment sums, then sums[alpha][4]
+  double *red = reinterpret_cast<double *>(dynLds), *segSum = red + (L * CELLS + 1) * NC, *sums = segSum + P.nSeg * NC;
+  typedef unsigned short E8 __attribute__((ext_vector_type(GAMMA_SEG)));
+  E8 ent = 0;
+  if (tid < P.nSeg) ent = *reinterpret_cast<const E8 *>(P.ent + GAMMA_SEG * tid);   // nSeg <= blockDim.x
+#pragma unroll
+  for (int k0 = 0; k0 < 4; k0 += NC) {
+    for (int g = 0; g < GR; g++) {
+      __syncthreads();
+      if (grp == g) {
+#pragma unroll
+        for (int l = 0; l < L; l++)
+#pragma unroll
+          for (int k = 0; k < NC; k++) {
+            double *d = red + (l * CELLS + cell) * NC + k;
+            *d = g ? *d + acc[l][k0 + k] : acc[l][k0 + k];
+          }
+      }
+    }
+    if (tid < NC) red[L * CELLS * NC + tid] = 0.0;
+    __syncthreads();
+    if (tid < P.nSeg) {
+      double v[NC] = {};
+#pragma unroll
+      for (int e = 0; e < GAMMA_SEG; e++)
+#pragma unroll
+        for (int k = 0; k < NC; k++) v[k] += red[ent[e] * NC + k];
+#pragma unroll
+      for (int k = 0; k < NC; k++) segSum[tid * NC + k] = v[k];
+    }
+    __syncthreads();
+    for (int i = tid; i < nm * NC; i += blockDim.x) {
+      const int a = i / NC, k = i % NC;
+      double v = 0.0;
+      for (int q = P.alphaSeg[a]; q < P.alphaSeg[a + 1]; q++) v += segSum[q * NC + k];
+      sums[a * 4 + k0 + k] = v;
+    }
+  }
+  __syncthreads();
+  constexpr int NO = TR || DK ? 2 : 4;
+  for (int a = tid; a < nmMax; a += blockDim.x) {
+    double v[NO] = {};
+    if (a < nm && a < C.nOut) {
+      const double t1 = sums[4 * a], t2 = sums[4 * a + 1], t3 = sums[4 * a + 2], t4 = sums[4 * a + 3];
       if constexpr (DK) {
         v[0] = t1;
         v[1] = t3;
@@ -2231,9 +2437,9 @@ __global__ __launch_bounds__(256) void k_l2lp(const R *__restrict__ Q0, const R 
 //   far[p] = sum_a M[a] u[a],  far[p + n] = sum_a M[a] (n . g[a]),  g_d[a] = v[a + e_d].
 // A wave takes four panels at a time, lanes over slots with u and g of their
 // slots in registers; the eight sums are reduced together, halving the values
-// with the lanes (10 exchanges instead of 48).  HBM bounds it (one column per
-// panel).  317k panels, order 6: 122 -> 119 us; 655k panels, order 8 (which had
-// no fused form: its partial sums did not fit in LDS): 1,715 -> 318 us.
+// with the lanes, by lane moves (through LDS exchanges the pass took 120 us).  HBM bounds it (one column per
+// panel).  317k panels, order 6: 122 -> 79 us; 655k panels, order 8 (which had no
+// fused form: its partial sums did not fit in LDS): 1,715 -> 228 us.
 // TR: the transposed M2M and Q2M of the adjoint operator, from the adjoint
 // moments (M_pot | M_dpdn): far[p] = N . M_pot, far[p + n] = M . M_dpdn.
 template <int V, int NL, bool TR>
@@ -2269,19 +2475,24 @@ __global__ __launch_bounds__(256) void k_l2lp64(const double *__restrict__ Q0, c
       f = f * tr / (k + 1);
     }
   }
-  const int i1 = mt.x & 0xff, i2 = (mt.x >> 8) & 0xff, i3 = (mt.x >> 16) & 0xff;
+  const int i1 = mt.x & 0xff;
   __syncthreads();
   for (int s = 1; s <= nUp; s++) {
     const int pin = O.p[s - 1], nIn = NMOM(pin), nOut = NMOM(O.p[s]);
     for (int d = 2; d >= 0; d--) {   // z, y, x
       const double *cd = co[s - 1][d];
       if (t < (d == 0 ? nOut : nIn)) {
+        // slots t + k e_d: from degree g to g + 1 the graded index grows by
+        // (g + 1)(g + 2)/2 + (z: i1, y: i1 + 1, x: g + 2)
         const int kmax = pin - deg_of(mt);
         double2 u = make_double2(0.0, 0.0);
-        for (int k = 0; k <= kmax; k++) {
-          const double2 v = cur[idx3(i1 + (d == 0 ? k : 0), i2 + (d == 1 ? k : 0), i3 + (d == 2 ? k : 0))];
+        for (int k = 0, i = t, g = deg_of(mt), tri = (g + 1) * (g + 2) / 2; k <= kmax; k++) {
+          const double2 v = cur[i];
           u.x += cd[k] * v.x;
           u.y += cd[k] * v.y;
+          i += tri + (d == 2 ? i1 : d == 1 ? i1 + 1 : g + 2);
+          tri += g + 2;
+          g++;
         }
         if (d == 0) {   // the kid's own M2L locals
           const double2 o = own[(s - 1) * nmMax + t];
@@ -2345,17 +2556,7 @@ __global__ __launch_bounds__(256) void k_l2lp64(const double *__restrict__ Q0, c
         v8[2 * k + 1] = t1;
       }
       if (j0 + 16 < cn) fetch(j0 + 16);   // in flight under the reduction
-#pragma unroll
-      for (int h = 4, o = 32; h > 0; h >>= 1, o >>= 1) {   // a lane keeps the half its bit o selects
-        const bool up = lane & o;
-#pragma unroll
-        for (int k = 0; k < h; k++) {
-          const double keep = up ? v8[k + h] : v8[k], give = up ? v8[k] : v8[k + h];
-          v8[k] = keep + __shfl_xor(give, o, 64);
-        }
-      }
-      double r = v8[0];
-      for (int o = 4; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
+      const double r = waveSum8(v8, lane);
       const int k = lane >> 4, which = (lane >> 3) & 1;
       if ((lane & 7) == 0 && j0 + k < cn) far[s0 + c0 + j0 + k + (which != (TR ? 1 : 0) ? n : 0)] = r;
     }
@@ -2934,7 +3135,7 @@ __global__ __launch_bounds__(64) void k_m2l_dk(const int *__restrict__ m2lOff, c
   if (tid == 0) part[c] = acc;
 }
 
-// the same sum from k_m2l_grid<DK>'s (t1, t3) per cube: part[c] =
+// the same sum from k_m2l_gamma<DK>'s (t1, t3) per cube: part[c] =
 // sum_a (eps a + b)[a] t1[a] - (a + b / eps)[a] t3[a], (b, a) the adjoint locals
 __global__ __launch_bounds__(64) void k_dk_far_dot(const int *__restrict__ cubeLevel, const int *__restrict__ ordMom,
                                                    const double *__restrict__ adjL, const double *__restrict__ t13,
@@ -4346,11 +4547,15 @@ struct fbh_ctx {
   // M2L term grid (k_m2l_grid): K steps x 64 lanes per order, runs of L steps
   int gridK = 0, gridL = 0, gridSlotZ = 0, gridNcc = 0, gridNgg = 0, gridWaves = 4;
   unsigned *gridTerms = nullptr;
-  int *m2lOrder = nullptr;     // cubes by interaction-list length, longest first (k_m2l_grid)
+  int *m2lOrder = nullptr;     // cubes by interaction-list length, longest first
+  int gmShape = -1, gmGroups = 1;   // the FP64 M2L by tensor slot (k_m2l_gamma): shape, groups per block
+  GammaPlans gmPlans = {};
+  GammaCube *gmCubes = nullptr;
+  size_t gmLds = 0;
   std::vector<int> hM2lOff;    // host copy of m2lOff
   int *gridOff = nullptr, *gridRedStart = nullptr;
   unsigned short *gridRedCell = nullptr;
-  size_t gridLds = 0, gridLds32 = 0;
+  size_t gridLds32 = 0;
   int ldsMax = 65536;
   // FP32 operator (precision form): copies of the cached operator in FP32
   bool fp32 = false;
@@ -4895,6 +5100,12 @@ static bool planGrid(const fbh_ctx *c, int p, int K, int L, int slotZ, std::vect
 // The term grid for every order the levels use, on the smallest compiled shape
 // (K, L) that holds the largest of them; none above order 8 (k_m2l_cached then).
 static bool buildM2LGrid(fbh_ctx *c) {
+  std::vector<int> order(c->nCube);   // cubes by interaction-list length, longest first
+  for (int i = 0; i < c->nCube; i++) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return c->hM2lOff[a + 1] - c->hM2lOff[a] > c->hM2lOff[b + 1] - c->hM2lOff[b];
+  });
+  if (!(c->m2lOrder = dupload(c, order.data(), order.size()))) return false;
   int pU = 0;
   for (int l = c->height; l <= c->depth; l++) pU = std::max(pU, c->ordM2L[l]);
   static const int shapes[][3] = {{3, 4, 1}, {5, 8, 1}, {6, 16, 2}, {7, 32, 4}, {8, 64, 8}};   // max order, K, L
@@ -4929,13 +5140,7 @@ static bool buildM2LGrid(fbh_ctx *c) {
   auto lds = [&](size_t elem) {
     return std::max((size_t)nw * (ncc + ngg) * 2 * elem, (size_t)(K / L) * 64 * 4 * elem);
   };
-  if (lds(sizeof(double)) > (size_t)c->ldsMax) return true;
-  std::vector<int> order(c->nCube);   // cubes by interaction-list length, longest first
-  for (int i = 0; i < c->nCube; i++) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    return c->hM2lOff[a + 1] - c->hM2lOff[a] > c->hM2lOff[b + 1] - c->hM2lOff[b];
-  });
-  if (!(c->m2lOrder = dupload(c, order.data(), order.size()))) return false;
+  if (lds(sizeof(float)) > (size_t)c->ldsMax) return true;
   if (!(c->gridTerms = dupload(c, allTerms.data(), allTerms.size())) ||
       !(c->gridOff = dupload(c, off.data(), off.size())) ||
       !(c->gridRedStart = dupload(c, allStart.data(), allStart.size())) ||
@@ -4946,9 +5151,142 @@ static bool buildM2LGrid(fbh_ctx *c) {
   c->gridSlotZ = nmU;
   c->gridNcc = ncc;
   c->gridNgg = ngg;
-  c->gridLds = lds(sizeof(double));
   c->gridLds32 = lds(sizeof(float));
   c->gridWaves = nw;
+  return true;
+}
+
+// k_m2l_gamma's compiled shapes: largest order, betas per cell L, waves per group W,
+// pairs per batch NB, sums per reduction round NC (a round's table within 32 KB,
+// so that LDS does not bound the resident blocks).  W x 64 lanes hold the cells of
+// the order (order 6: 250 of 256 at L = 4, 90 % of the steps busy; order 8: 505 of
+// 512 at L = 7, 84 %).
+static constexpr int kGamma[][5] = {{3, 2, 1, 4, 4}, {4, 4, 1, 4, 4}, {5, 2, 4, 4, 4}, {6, 4, 4, 4, 4}, {7, 4, 8, 4, 2}, {8, 7, 8, 4, 1}};
+
+// The cells of order p: every product (gamma, beta <= gamma) dealt into cells of at
+// most L betas of one gamma, consecutive gammas on consecutive lanes (the tensor
+// loads stay coalesced), and per step the beta that clashes least with the lanes
+// already placed in its group of 16 (LDS serves 16 lanes' 16-byte slots at a time,
+// slot mod 16 picks the banks, equal slots are broadcast).
+struct HostGamma {
+  std::vector<int> gamma, alphaSeg;
+  std::vector<unsigned short> beta, ent;
+};
+static bool planGamma(int p, int L, int W, int slotZ, HostGamma &H) {
+  const int nm = NMOM(p), cells = 64 * W;
+  std::vector<int> mi(3 * nm);
+  for (int d = 0, g = 0; d <= p; d++)
+    for (int i1 = 0; i1 <= d; i1++)
+      for (int i2 = 0; i2 <= d - i1; i2++, g++) {
+        mi[3 * g] = i1;
+        mi[3 * g + 1] = i2;
+        mi[3 * g + 2] = d - i1 - i2;
+      }
+  std::vector<std::vector<int>> pool(nm);
+  std::vector<int> size;
+  H.gamma.clear();
+  for (int g = 0; g < nm; g++) {
+    for (int b = 0; b < nm; b++)
+      if (mi[3 * b] <= mi[3 * g] && mi[3 * b + 1] <= mi[3 * g + 1] && mi[3 * b + 2] <= mi[3 * g + 2]) pool[g].push_back(b);
+    const int m = (int)pool[g].size(), k = (m + L - 1) / L;
+    for (int i = 0; i < k; i++) {   // even shares
+      H.gamma.push_back(g);
+      size.push_back(m / k + (i < m % k));
+    }
+  }
+  if ((int)H.gamma.size() > cells) return false;
+  const int used = (int)H.gamma.size();
+  H.gamma.resize(cells, 0);
+  size.resize(cells, 0);
+  H.beta.assign((size_t)L * cells, (unsigned short)slotZ);
+  std::vector<std::vector<int>> byAlpha(nm);
+  std::vector<int> at(cells);
+  for (int l = 0; l < L; l++) {
+    std::fill(at.begin(), at.end(), -1);
+    for (int i = 0; i < used; i++) {
+      if (size[i] <= l) continue;
+      auto &pl = pool[H.gamma[i]];
+      size_t best = 0;
+      int bc = 1 << 30;
+      for (size_t q = 0; q < pl.size() && bc > 0; q++) {
+        int n = 0;
+        for (int j = i / 16 * 16; j < i; j++)
+          if (at[j] >= 0 && at[j] != pl[q] && at[j] % 16 == pl[q] % 16) n++;
+        if (n < bc) { bc = n; best = q; }
+      }
+      const int b = at[i] = pl[best], g = H.gamma[i];
+      pl.erase(pl.begin() + best);
+      H.beta[(size_t)l * cells + i] = (unsigned short)b;
+      byAlpha[idx3of(mi[3 * g] - mi[3 * b], mi[3 * g + 1] - mi[3 * b + 1], mi[3 * g + 2] - mi[3 * b + 2])].push_back(l * cells + i);
+    }
+  }
+  H.alphaSeg.assign(1, 0);
+  H.ent.clear();
+  for (int a = 0; a < nm; a++) {
+    for (int e : byAlpha[a]) H.ent.push_back((unsigned short)e);
+    while (H.ent.size() % GAMMA_SEG) H.ent.push_back((unsigned short)(L * cells));
+    H.alphaSeg.push_back((int)H.ent.size() / GAMMA_SEG);
+  }
+  return true;
+}
+
+// The plans of every order the levels use, on the smallest compiled shape that
+// holds the largest (none above order 8: k_m2l_cached).
+static bool buildGamma(fbh_ctx *c) {
+  int pU = 0;
+  for (int l = c->height; l <= c->depth; l++) pU = std::max(pU, c->ordM2L[l]);
+  const char *em = getenv("FABIPB_M2L");   // "items": the item-list kernel only (check path)
+  if (em && !strcmp(em, "items")) return true;
+  int sh = -1;
+  for (int i = 0; i < (int)(sizeof(kGamma) / sizeof(kGamma[0])) && sh < 0; i++)
+    if (pU <= kGamma[i][0]) sh = i;
+  if (sh < 0) return true;
+  const int L = kGamma[sh][1], W = kGamma[sh][2], NB = kGamma[sh][3], NC = kGamma[sh][4], nmU = NMOM(kGamma[sh][0]);
+  size_t redLen = 0;
+  int maxSeg = 0;
+  for (int l = c->height; l <= c->depth; l++) {
+    const int p = c->ordM2L[l];
+    GammaPlan &P = c->gmPlans.p[p];
+    if (P.gamma) continue;
+    HostGamma H;
+    if (!planGamma(p, L, W, nmU, H)) return true;
+    // one upload: ent first (16-byte loads), then beta, gamma, alphaSeg
+    std::vector<unsigned short> all(H.ent);
+    all.insert(all.end(), H.beta.begin(), H.beta.end());
+    const size_t oI = all.size();   // even: both lengths are multiples of 8
+    all.resize(oI + 2 * (H.gamma.size() + H.alphaSeg.size()));
+    memcpy(&all[oI], H.gamma.data(), H.gamma.size() * sizeof(int));
+    memcpy(&all[oI + 2 * H.gamma.size()], H.alphaSeg.data(), H.alphaSeg.size() * sizeof(int));
+    const unsigned short *d = dupload(c, all.data(), all.size());
+    if (!d) return false;
+    P.ent = d;
+    P.beta = d + H.ent.size();
+    P.gamma = reinterpret_cast<const int *>(d + oI);
+    P.alphaSeg = P.gamma + H.gamma.size();
+    P.nSeg = H.alphaSeg.back();
+    maxSeg = std::max(maxSeg, P.nSeg);
+    redLen = std::max(redLen, ((size_t)L * 64 * W + 1) * NC + (size_t)P.nSeg * NC + 4 * (size_t)NMOM(p));
+  }
+  // groups per block: four one-wave groups at the small orders; two four-wave
+  // groups while the cubes alone leave CUs idle (1,280 panels: 28 -> 21 us)
+  const int gr = W == 1 ? 4 : W == 4 && c->nCube < 1024 ? 2 : 1;
+  const size_t lds = std::max((size_t)gr * 4 * NB * (nmU + 1) * sizeof(double2), redLen * sizeof(double));
+  if (lds > (size_t)c->ldsMax || maxSeg > 64 * W * gr) return true;
+  std::vector<GammaCube> cubes(c->nCube);   // longest interaction lists first
+  for (int i = 0; i < c->nCube; i++) cubes[i].cube = i;
+  std::stable_sort(cubes.begin(), cubes.end(), [&](const GammaCube &a, const GammaCube &b) {
+    return c->hM2lOff[a.cube + 1] - c->hM2lOff[a.cube] > c->hM2lOff[b.cube + 1] - c->hM2lOff[b.cube];
+  });
+  for (GammaCube &q : cubes) {
+    q.b0 = c->hM2lOff[q.cube];
+    q.b1 = c->hM2lOff[q.cube + 1];
+    q.p = c->ordM2L[c->cubeLevel[q.cube]];
+    q.nOut = NMOM(c->ordMom[c->cubeLevel[q.cube]]);
+  }
+  if (!(c->gmCubes = dupload(c, cubes.data(), cubes.size()))) return false;
+  c->gmShape = sh;
+  c->gmGroups = gr;
+  c->gmLds = lds;
   return true;
 }
 
@@ -5227,7 +5565,7 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
   }
   // M2L derivative tensors per pair, cached when they fit (1344 B per pair at p=6)
   c->m2lG = nullptr;
-  if (!buildM2LPlan(c) || !buildM2LGrid(c)) FAIL();
+  if (!buildM2LPlan(c) || !buildM2LGrid(c) || !buildGamma(c)) FAIL();
   if (c->m2lWaves > 0 && c->nM2L > 0 && (double)c->nM2L * 2 * c->nmMax * sizeof(double) <= M2L_CACHE_BYTES) {
     std::vector<int> pd((size_t)c->nM2L);
     for (int cb = 0; cb < nCube; cb++)
@@ -5246,7 +5584,7 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
     // leaves' spheres about their cube centres
     std::vector<double> rad(nLeaf, 0.0);
     const double t = c->Q.t[0];
-    bool ok = true;
+    double sum = 0.0;
     for (int l = 0; l < nLeaf; l++)
       for (int j = leafStart[l]; j < leafStart[l] + leafCount[l]; j++) {
         double d2 = 0.0;
@@ -5254,9 +5592,11 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
           const double d = hp[j].v[k] + t * (hp[j].a[6 + k] + t * hp[j].a[k]) - cubeX[3 * l + k];
           d2 += d * d;
         }
-        if (!std::isfinite(d2)) ok = false;
-        rad[l] = std::max(rad[l], std::sqrt(d2));
+        sum += d2;
+        rad[l] = std::max(rad[l], d2);
       }
+    const bool ok = std::isfinite(sum);
+    for (double &r : rad) r = std::sqrt(r);
     double rMax = 1.0;   // a panel against itself is evaluated at r = 1 with zero weight
     for (int l = 0; l < nLeaf; l++)
       for (int k = nearOff[l]; k < nearOff[l + 1]; k++) {
@@ -5292,33 +5632,56 @@ static void m2lLaunch(fbh_ctx *c, const OpBufs<R> &B, hipStream_t st) {
                      c->planTerms, c->planIdx, c->planOff);
 }
 
-template <typename R, int K, int L, bool TR = false, bool DK = false>
-static void m2lGridLaunch(fbh_ctx *c, const R *G, const R *mom, R *lec, size_t lds, hipStream_t st) {
-  hipLaunchKernelGGL((k_m2l_grid<R, K, L, TR, DK>), dim3(c->nCube), dim3(64 * c->gridWaves), lds, st, c->m2lOff,
+template <int K, int L>
+static void m2lGridLaunch(fbh_ctx *c, const float *G, const float *mom, float *lec, hipStream_t st) {
+  hipLaunchKernelGGL((k_m2l_grid<float, K, L>), dim3(c->nCube), dim3(64 * c->gridWaves), c->gridLds32, st, c->m2lOff,
                      c->m2lSrc,
-                     c->cubeLevelD, c->ordM2LD, c->ordMomD, G, mom, lec, c->nmMax, (R)c->eps, c->T, c->gridTerms,
+                     c->cubeLevelD, c->ordM2LD, c->ordMomD, G, mom, lec, c->nmMax, (float)c->eps, c->T, c->gridTerms,
                      c->gridOff, c->gridRedStart, c->gridRedCell, c->gridSlotZ, c->gridNcc, c->gridNgg,
                      c->m2lOrder);
 }
 
-// k_m2l_grid at the shape the plan was built for; false when there is no grid
-template <typename R, bool TR = false, bool DK = false>
-static bool m2lGrid(fbh_ctx *c, const R *G, const R *mom, R *lec, hipStream_t st) {
+// k_m2l_grid (FP32) at the shape the plan was built for; false when there is no grid
+static bool m2lGrid(fbh_ctx *c, const float *G, const float *mom, float *lec, hipStream_t st) {
   if (!c->gridK || !G) return false;
-  const size_t lds = sizeof(R) == sizeof(double) ? c->gridLds : c->gridLds32;
   switch (c->gridK) {
-    case 4: m2lGridLaunch<R, 4, 1, TR, DK>(c, G, mom, lec, lds, st); return true;
-    case 8: m2lGridLaunch<R, 8, 1, TR, DK>(c, G, mom, lec, lds, st); return true;
-    case 16: m2lGridLaunch<R, 16, 2, TR, DK>(c, G, mom, lec, lds, st); return true;
-    case 32: m2lGridLaunch<R, 32, 4, TR, DK>(c, G, mom, lec, lds, st); return true;
-    case 64: m2lGridLaunch<R, 64, 8, TR, DK>(c, G, mom, lec, lds, st); return true;
+    case 4: m2lGridLaunch<4, 1>(c, G, mom, lec, st); return true;
+    case 8: m2lGridLaunch<8, 1>(c, G, mom, lec, st); return true;
+    case 16: m2lGridLaunch<16, 2>(c, G, mom, lec, st); return true;
+    case 32: m2lGridLaunch<32, 4>(c, G, mom, lec, st); return true;
+    case 64: m2lGridLaunch<64, 8>(c, G, mom, lec, st); return true;
+  }
+  return false;
+}
+
+template <int S, bool TR, bool DK>
+static void m2lGammaLaunch(fbh_ctx *c, const double *G, const double *mom, double *lec, hipStream_t st) {
+  constexpr int PM = kGamma[S][0], L = kGamma[S][1], W = kGamma[S][2], NB = kGamma[S][3], NC = kGamma[S][4];
+  hipLaunchKernelGGL((k_m2l_gamma<PM, L, W, NB, NC, TR, DK>), dim3(c->nCube), dim3(64 * W * c->gmGroups), c->gmLds, st,
+                     c->gmCubes, c->m2lSrc, G, mom, lec, c->nmMax, c->eps, c->T, c->gmPlans);
+}
+// k_m2l_gamma (FP64) at the shape the plans were built for; false when there are none
+template <bool TR = false, bool DK = false>
+static bool m2lGamma(fbh_ctx *c, const double *G, const double *mom, double *lec, hipStream_t st) {
+  if (!G) return false;
+  switch (c->gmShape) {
+    case 0: m2lGammaLaunch<0, TR, DK>(c, G, mom, lec, st); return true;
+    case 1: m2lGammaLaunch<1, TR, DK>(c, G, mom, lec, st); return true;
+    case 2: m2lGammaLaunch<2, TR, DK>(c, G, mom, lec, st); return true;
+    case 3: m2lGammaLaunch<3, TR, DK>(c, G, mom, lec, st); return true;
+    case 4: m2lGammaLaunch<4, TR, DK>(c, G, mom, lec, st); return true;
+    case 5: m2lGammaLaunch<5, TR, DK>(c, G, mom, lec, st); return true;
   }
   return false;
 }
 
 template <typename R>
 static void m2lPass(fbh_ctx *c, const OpBufs<R> &B, hipStream_t st) {
-  if (m2lGrid<R>(c, B.G, B.mom, B.lec, st)) return;
+  if constexpr (std::is_same<R, double>::value) {
+    if (m2lGamma(c, B.G, B.mom, B.lec, st)) return;
+  } else {
+    if (m2lGrid(c, B.G, B.mom, B.lec, st)) return;
+  }
   if (B.G) {
     if (c->m2lMaxT == 16) m2lLaunch<R, 16>(c, B, st);
     else if (c->m2lMaxT == 32) m2lLaunch<R, 32>(c, B, st);
@@ -5620,7 +5983,7 @@ static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
                        c->cubeLevelD, c->ordM2LD, c->ordMomD, (const double *)c->m2lG, (const double *)c->adjL,
                        c->adjM, c->nmMax, c->eps, c->T, c->planTerms, c->planIdx, c->planOff);
   };
-  if (m2lGrid<double, true>(c, c->m2lG, c->adjL, c->adjM, st)) {
+  if (m2lGamma<true>(c, c->m2lG, c->adjL, c->adjM, st)) {
   } else if (c->m2lMaxT == 16) launch(k_m2l_cached<double, 16, true>);
   else if (c->m2lMaxT == 32) launch(k_m2l_cached<double, 32, true>);
   else launch(k_m2l_cached<double, 0, true>);
@@ -6775,13 +7138,13 @@ static int kappaOperatorTerms(fbh_ctx *c, const double *sgm_dev, const double *l
     B.mom = c->adjL;
     for (int lev = c->depth - 1; lev >= c->height; lev--)
       if (!m2mAxPass(c, B, lev, c->stream)) m2mPass(c, B, lev, c->stream);
-    if (c->gridK && c->m2lG && !c->m2lGdk) {   // (dGk/dkappa, Gk) per pair, cached as the M2L tensors are
+    if (c->gmShape >= 0 && c->m2lG && !c->m2lGdk) {   // (dGk/dkappa, Gk) per pair, cached as the M2L tensors are
       if (!(c->m2lGdk = dalloc<double>(c, (size_t)c->nM2L * 2 * c->nmMax))) return 0;
       hipLaunchKernelGGL(k_m2l_derivs, dim3((unsigned)c->nM2L), dim3(64),
                          2 * (size_t)derivScratch(c->maxOrder) * sizeof(double), c->stream, c->m2lDst, c->m2lSrc,
                          c->cubeLevelD, c->ordM2LD, c->cubeX, c->m2lGdk, c->nmMax, c->kappa, c->T, true);
     }
-    if (c->m2lGdk && m2lGrid<double, false, true>(c, c->m2lGdk, c->mom, c->lec, c->stream)) {
+    if (c->m2lGdk && m2lGamma<false, true>(c, c->m2lGdk, c->mom, c->lec, c->stream)) {
       hipLaunchKernelGGL(k_dk_far_dot, dim3(c->nCube), dim3(64), 0, c->stream, c->cubeLevelD, c->ordMomD, c->adjL,
                          c->lec, part, c->nmMax, c->eps);
     } else {
