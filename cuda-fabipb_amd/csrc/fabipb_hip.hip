@@ -3463,7 +3463,8 @@ __device__ inline void rhsDirect(const double *qp, const double *nr, const doubl
 //   sum_g r^g sum_j (n . V[g][j]) (eps Gk - G0)_(|g|+j)
 // W and V depend on the cluster only, so they are formed once per cluster
 // (k_ct_poly) and every point evaluates a fixed, unrolled polynomial.
-// Entry order (k_ct_poly and enFar agree on it): W then V; g1 descending,
+// Entry order (k_ct_poly, enFar64 and enFar32 agree on it): W (all the FP64 walk
+// reads) then V; g1 descending,
 // g2 descending, g3 descending (the Horner order), then j; a V entry holds
 // three values.
 
@@ -3535,28 +3536,40 @@ __global__ __launch_bounds__(256) void k_ct_poly(int c0, const double *__restric
 // per order: the largest chunk that leaves the scalar registers unspilled
 // (counted in the compiled code: 32 at orders 6 and 7, 8 elsewhere)
 __host__ __device__ constexpr int enChunk(int p) { return EN_CHUNK >= 0 ? EN_CHUNK : (p == 6 || p == 7) ? 32 : 8; }
+// The FP64 far term from the W table alone.  With A(r) = sum_g r^g sum_j W[g][j]
+// u_(|g|+j) the far potential of the kernel u, its normal derivative is
+//   n . grad A = sum_g (n . grad r^g) sum_j W[g][j] u_(|g|+j) + sum_g r^g sum_j W[g][j] (n.r) u_(|g|+j+1)
+// (f_k = ((1/r) d/dr)^k f, so grad f_k = r f_(k+1)): a Horner scheme that carries
+// the value and the derivative along n, the second sum entering the derivative's
+// coefficients.  Against the separate V table of the normal derivative (three
+// values an entry; the FP32 walk's form) that is 866 FMAs and 130 doubles a cluster
+// instead of 1,134 and 730 at order 6, 1,765 and 295 instead of 2,360 and 1,555 at
+// order 8; the right-hand side, whose two kernels are the same, drops the first
+// sum as well (596 and 1,140).  Tree right-hand side and energy together, 163,840
+// panels at order 8: 7.96 -> 3.39 ms.
 // MODE 0: the energy's kernels G0 - Gk and eps Gk - G0 (src/treecode.c:581-615);
 // MODE 1: the right-hand side's Coulomb kernel 1/r (:283-379), both halves;
 // MODE 3: d/dkappa of MODE 0's kernels; MODE 4: MODE 0 into (y0, y1) and
-// MODE 3 into (z0, z1) from one pass over the coefficients
-// R: the type of the coefficients and of the polynomial's arithmetic (float for
-// the precision form's energy: half the scalar-load bytes per cluster; the
-// radial values are formed in FP64 and rounded, the sums return to FP64)
-template <int P, int MODE, typename R = double>
-__device__ __forceinline__ void enFar(const R *__restrict__ co0, double rxd, double ryd, double rzd, double nxd,
-                                      double nyd, double nzd, double kappa, double eps, double &y0, double &y1,
-                                      double &z0, double &z1) {
+// MODE 3 into (z0, z1) from one pass over the coefficients.
+// Nested Horner in x (outer), y, z (inner).  The coefficients are wave-uniform
+// and come in through scalar loads in chunks of (a, b) rows of at least
+// enChunk(P) doubles: after a chunk an empty asm takes the table pointer and the
+// running sums, so the next chunk's loads cannot be issued before this chunk is
+// consumed (hoisted all at once, they overflow the scalar registers and are
+// spilled).
+template <int P, int MODE>
+__device__ __forceinline__ void enFar64(const double *__restrict__ co0, double rx, double ry, double rz, double nx,
+                                        double ny, double nz, double kappa, double eps, double &y0, double &y1,
+                                        double &z0, double &z1) {
   constexpr int NS = MODE == 4 ? 2 : 1;   // radial sequence pairs evaluated together
-  const double rho = sqrt(rxd * rxd + ryd * ryd + rzd * rzd);
-  const R rx = (R)rxd, ry = (R)ryd, rz = (R)rzd, nx = (R)nxd, ny = (R)nyd, nz = (R)nzd;
-  double h[NS][P + 2], u[NS][P + 2];
+  constexpr bool SAME = MODE == 1;        // u = h
+  const double rho = sqrt(rx * rx + ry * ry + rz * rz), nr = nx * rx + ny * ry + nz * rz;
+  double h[NS][P + 2], u[NS][P + 2], v[NS][P + 1];   // v_k = (n.r) u_(k+1)
   if constexpr (MODE == 1) {
     const double nr2 = -1.0 / (rho * rho);
-    h[0][0] = 1.0 / rho;
+    u[0][0] = 1.0 / rho;
 #pragma unroll
-    for (int k = 0; k <= P; k++) h[0][k + 1] = (2 * k + 1) * nr2 * h[0][k];
-#pragma unroll
-    for (int k = 0; k <= P + 1; k++) u[0][k] = h[0][k];
+    for (int k = 0; k <= P; k++) u[0][k + 1] = (2 * k + 1) * nr2 * u[0][k];
   } else {
     double g0[P + 2], gk[P + 2];
     radial(kappa, rho, P + 1, g0, 1, gk, 1);
@@ -3578,107 +3591,148 @@ __device__ __forceinline__ void enFar(const R *__restrict__ co0, double rxd, dou
       }
     }
   }
-  // nested Horner in x (outer), y, z (inner); a coefficient of r^g is the
-  // j-sum over the radial values of degree |g| + j.  The coefficients are
-  // wave-uniform and come in through scalar loads in chunks of (a, b) rows of
-  // at least enChunk(P) doubles: after a chunk an empty asm takes the table
-  // pointer and the running sums, so the next chunk's loads cannot be issued
-  // before this chunk is consumed (hoisted all at once, they overflow the
-  // scalar registers and are spilled).
-  using CD = const __attribute__((address_space(4))) R;
-  CD *co = (CD *)co0;
-  constexpr int CHUNK = enChunk(P) * (int)(sizeof(double) / sizeof(R));   // the same bytes per chunk
-  R hr[NS][P + 2], ur[NS][P + 2];
 #pragma unroll
   for (int t = 0; t < NS; t++)
 #pragma unroll
-    for (int k = 0; k <= P + 1; k++) {
-      hr[t][k] = (R)h[t][k];
-      ur[t][k] = (R)u[t][k];
-    }
+    for (int k = 0; k <= P; k++) v[t][k] = nr * u[t][k + 1];
+  using CD = const __attribute__((address_space(4))) double;
+  CD *co = (CD *)co0;
+  constexpr int CHUNK = enChunk(P);
   int o = 0, since = 0;   // since: coefficients read since the last chunk boundary
-  R s0[NS], s1[NS];
-#pragma unroll
-  for (int t = 0; t < NS; t++) s0[t] = s1[t] = 0;
+  double sA[NS], sD[NS], sB[NS];   // value, derivative along n, value of the other kernel
 #pragma unroll
   for (int a = P; a >= 0; a--) {
-    R qa[NS];
-#pragma unroll
-    for (int t = 0; t < NS; t++) qa[t] = 0;
+    double qA[NS], qD[NS], qB[NS];
 #pragma unroll
     for (int b = P - a; b >= 0; b--) {
-      R rb[NS];
-#pragma unroll
-      for (int t = 0; t < NS; t++) rb[t] = 0;
+      double rA[NS], rD[NS], rB[NS];
 #pragma unroll
       for (int c = P - a - b; c >= 0; c--) {
         const int d = a + b + c;
+        const bool first = c == P - a - b;   // folds at compile time, as every test on a, b, c
 #pragma unroll
         for (int t = 0; t < NS; t++) {
-          R cw = 0;
+          double D = first ? 0.0 : fma(rD[t], rz, rA[t] * nz), A = first ? 0.0 : rA[t] * rz,
+                 B = first ? 0.0 : rB[t] * rz;
 #pragma unroll
-          for (int j = 0; j <= (P - d) / 2; j++) cw += hr[t][d + j] * co[o + j];
-          rb[t] = rb[t] * rz + cw;
+          for (int j = 0; j <= (P - d) / 2; j++) {
+            const double w = co[o + j];
+            D = first && j == 0 ? w * v[t][d] : fma(w, v[t][d + j], D);
+            A = first && j == 0 ? w * u[t][d] : fma(w, u[t][d + j], A);
+            if constexpr (!SAME) B = first && j == 0 ? w * h[t][d] : fma(w, h[t][d + j], B);
+          }
+          rD[t] = D;
+          rA[t] = A;
+          rB[t] = B;
         }
         o += (P - d) / 2 + 1;
         since += (P - d) / 2 + 1;
       }
 #pragma unroll
-      for (int t = 0; t < NS; t++) qa[t] = qa[t] * ry + rb[t];
+      for (int t = 0; t < NS; t++) {
+        const bool first = b == P - a;
+        qD[t] = first ? rD[t] : fma(qD[t], ry, fma(qA[t], ny, rD[t]));
+        qA[t] = first ? rA[t] : fma(qA[t], ry, rA[t]);
+        if constexpr (!SAME) qB[t] = first ? rB[t] : fma(qB[t], ry, rB[t]);
+      }
       if (CHUNK > 0 && since >= CHUNK) {   // folds at compile time
-        if constexpr (NS == 1)
-          asm volatile("" : "+s"(co), "+v"(qa[0]));
+        if constexpr (SAME)
+          asm volatile("" : "+s"(co), "+v"(qA[0]), "+v"(qD[0]));
+        else if constexpr (NS == 1)
+          asm volatile("" : "+s"(co), "+v"(qA[0]), "+v"(qD[0]), "+v"(qB[0]));
         else
-          asm volatile("" : "+s"(co), "+v"(qa[0]), "+v"(qa[1]));
+          asm volatile("" : "+s"(co), "+v"(qA[0]), "+v"(qD[0]), "+v"(qB[0]), "+v"(qA[1]), "+v"(qD[1]), "+v"(qB[1]));
         since = 0;
       }
     }
 #pragma unroll
-    for (int t = 0; t < NS; t++) s0[t] = s0[t] * rx + qa[t];
+    for (int t = 0; t < NS; t++) {
+      const bool first = a == P;
+      sD[t] = first ? qD[t] : fma(sD[t], rx, fma(sA[t], nx, qD[t]));
+      sA[t] = first ? qA[t] : fma(sA[t], rx, qA[t]);
+      if constexpr (!SAME) sB[t] = first ? qB[t] : fma(sB[t], rx, qB[t]);
+    }
+  }
+  y0 += SAME ? sA[0] : sB[0];
+  y1 += sD[0];
+  if constexpr (NS == 2) {
+    z0 += sB[1];
+    z1 += sD[1];
+  }
+}
+
+// The precision form's far term (the energy's kernels, MODE 0): coefficients and
+// polynomials in FP32 (half the scalar-load bytes per cluster; the radial values
+// are formed in FP64 and rounded, the sums return to FP64), from the W and V tables.
+template <int P>
+__device__ __forceinline__ void enFar32(const float *__restrict__ co0, double rxd, double ryd, double rzd, double nxd,
+                                        double nyd, double nzd, double kappa, double eps, double &y0, double &y1) {
+  const double rho = sqrt(rxd * rxd + ryd * ryd + rzd * rzd);
+  const float rx = (float)rxd, ry = (float)ryd, rz = (float)rzd, nx = (float)nxd, ny = (float)nyd, nz = (float)nzd;
+  double g0[P + 2], gk[P + 2];
+  radial(kappa, rho, P + 1, g0, 1, gk, 1);
+  float hr[P + 2], ur[P + 2];
+#pragma unroll
+  for (int k = 0; k <= P + 1; k++) {
+    hr[k] = (float)(g0[k] - gk[k]);
+    ur[k] = (float)(eps * gk[k] - g0[k]);
+  }
+  using CD = const __attribute__((address_space(4))) float;
+  CD *co = (CD *)co0;
+  constexpr int CHUNK = 2 * enChunk(P);   // the same bytes per chunk as enFar64
+  int o = 0, since = 0;
+  float s0 = 0, s1 = 0;
+#pragma unroll
+  for (int a = P; a >= 0; a--) {
+    float qa = 0;
+#pragma unroll
+    for (int b = P - a; b >= 0; b--) {
+      float rb = 0;
+#pragma unroll
+      for (int c = P - a - b; c >= 0; c--) {
+        const int d = a + b + c;
+        float cw = 0;
+#pragma unroll
+        for (int j = 0; j <= (P - d) / 2; j++) cw += hr[d + j] * co[o + j];
+        rb = rb * rz + cw;
+        o += (P - d) / 2 + 1;
+        since += (P - d) / 2 + 1;
+      }
+      qa = qa * ry + rb;
+      if (CHUNK > 0 && since >= CHUNK) {
+        asm volatile("" : "+s"(co), "+v"(qa));
+        since = 0;
+      }
+    }
+    s0 = s0 * rx + qa;
   }
 #pragma unroll
   for (int a = P + 1; a >= 0; a--) {
-    R qa[NS];
-#pragma unroll
-    for (int t = 0; t < NS; t++) qa[t] = 0;
+    float qa = 0;
 #pragma unroll
     for (int b = P + 1 - a; b >= 0; b--) {
-      R rb[NS];
-#pragma unroll
-      for (int t = 0; t < NS; t++) rb[t] = 0;
+      float rb = 0;
 #pragma unroll
       for (int c = P + 1 - a - b; c >= 0; c--) {
         const int d = a + b + c;
+        float cv = 0;
 #pragma unroll
-        for (int t = 0; t < NS; t++) {
-          R cv = 0;
-#pragma unroll
-          for (int j = 0; j <= (P + 1 - d) / 2; j++)
-            cv += ur[t][d + j] * (nx * co[o + 3 * j] + ny * co[o + 3 * j + 1] + nz * co[o + 3 * j + 2]);
-          rb[t] = rb[t] * rz + cv;
-        }
+        for (int j = 0; j <= (P + 1 - d) / 2; j++)
+          cv += ur[d + j] * (nx * co[o + 3 * j] + ny * co[o + 3 * j + 1] + nz * co[o + 3 * j + 2]);
+        rb = rb * rz + cv;
         o += 3 * ((P + 1 - d) / 2 + 1);
         since += 3 * ((P + 1 - d) / 2 + 1);
       }
-#pragma unroll
-      for (int t = 0; t < NS; t++) qa[t] = qa[t] * ry + rb[t];
-      if (CHUNK > 0 && since >= CHUNK) {   // folds at compile time
-        if constexpr (NS == 1)
-          asm volatile("" : "+s"(co), "+v"(qa[0]));
-        else
-          asm volatile("" : "+s"(co), "+v"(qa[0]), "+v"(qa[1]));
+      qa = qa * ry + rb;
+      if (CHUNK > 0 && since >= CHUNK) {
+        asm volatile("" : "+s"(co), "+v"(qa));
         since = 0;
       }
     }
-#pragma unroll
-    for (int t = 0; t < NS; t++) s1[t] = s1[t] * rx + qa[t];
+    s1 = s1 * rx + qa;
   }
-  y0 += (double)s0[0];
-  y1 += (double)s1[0];
-  if constexpr (NS == 2) {
-    z0 += (double)s0[1];
-    z1 += (double)s1[1];
-  }
+  y0 += (double)s0;
+  y1 += (double)s1;
 }
 
 // Panel-tree energy (src/treecode.c:617-695, 581-615; MODE 0), its weight
@@ -3698,12 +3752,14 @@ __device__ __forceinline__ void enFar(const R *__restrict__ co0, double rxd, dou
 #ifndef EN_TARGET_WAVES
 #define EN_TARGET_WAVES 8192   // slices are added until the walk has this many waves
 #endif
-// waves per SIMD the walk's registers must allow: 4 for the energy's modes (a
-// few spilled registers; 2.5 against 2.8 ms with three waves at 317k panels),
-// the compiler's choice for the right-hand side (five waves) and MODE 4
-__host__ __device__ constexpr int enMinWaves(int mode) { return mode == 0 || mode == 2 || mode == 3 ? 4 : 1; }
+// waves per SIMD the walk's registers must allow: 4 (a few spilled registers in
+// the energy's modes), 3 for those at orders 8 and 9 (53 and 67 spills at four),
+// the compiler's choice for MODE 4
+__host__ __device__ constexpr int enMinWaves(int mode, int p) {
+  return mode == 4 ? 1 : mode != 1 && p >= 8 ? 3 : 4;
+}
 template <int P, int MODE, typename R = double>
-__global__ __launch_bounds__(64 * EN_WPB, enMinWaves(MODE)) void k_energy_wave(const Pnl *__restrict__ pnl, int n, const double *__restrict__ sgm,
+__global__ __launch_bounds__(64 * EN_WPB, enMinWaves(MODE, P)) void k_energy_wave(const Pnl *__restrict__ pnl, int n, const double *__restrict__ sgm,
                                                      const int *__restrict__ level, const double *__restrict__ cx,
                                                      const double *__restrict__ eRad,
                                                      const int *__restrict__ kidStart, const int *__restrict__ nKids,
@@ -3765,9 +3821,13 @@ __global__ __launch_bounds__(64 * EN_WPB, enMinWaves(MODE)) void k_energy_wave(c
         const bool acc = on && eRad[cb] < theta * dist && lev >= height;
         const bool dir = on && !acc && lev == depth;
         const unsigned long long down = __ballot(on && !acc && lev < depth);
-        if (acc)
-          enFar<P, MODE == 2 ? 0 : MODE, R>(poly + (long long)(cb - c0) * SZ, rx, ry, rz, nr[0], nr[1], nr[2], kappa, eps,
-                                         y0, y1, z0, z1);
+        if (acc) {
+          if constexpr (std::is_same<R, float>::value)
+            enFar32<P>(poly + (long long)(cb - c0) * SZ, rx, ry, rz, nr[0], nr[1], nr[2], kappa, eps, y0, y1);
+          else
+            enFar64<P, MODE == 2 ? 0 : MODE>(poly + (long long)(cb - c0) * SZ, rx, ry, rz, nr[0], nr[1], nr[2], kappa,
+                                             eps, y0, y1, z0, z1);
+        }
         if (__ballot(dir) != 0ull) {
           const int s = chgStart[cb], nq = nChgs[cb];
           for (int k = 0; k < nq; k++) {
@@ -4485,7 +4545,7 @@ struct ChargeSet {
   bool ready = false;
   // the cluster moments (and walk coefficients) of the staged charges are built:
   // they depend on the charges alone, so later walks of the same set reuse them
-  mutable bool momReady = false;
+  mutable bool momReady = false, polyReady32 = false;   // polyReady32: the FP32 walk's tables too
   int nChar = 0, nc = 0, c0 = -1, P = 0, S = 1, SZ = 0, nClus = 0, nDesc = 0;
   bool uni = false;
   std::vector<int> lvStart, lvCount, ord;
@@ -7351,16 +7411,22 @@ static int walkCharges(fbh_ctx *c, const ChargeSet &s, int mode, double theta, c
       hipLaunchKernelGGL(k_ct_m2m, dim3(lvCount[l]), dim3(blk64((nOut + 3) / 4, 256)), lds, strm, lvStart[l],
                          s.dKid, s.dNK, s.dX, s.dOrd, l, s.dMom, nmMax, c->T);
     }
-    if (s.uni) {
-      hipLaunchKernelGGL(k_ct_poly, dim3(s.nClus), dim3(256), 0, strm, s.c0, s.dMom, nmMax, s.dDesc, s.nDesc,
+    if (s.uni)   // the first enPolyW entries are the W table
+      hipLaunchKernelGGL(k_ct_poly, dim3(s.nClus), dim3(256), 0, strm, s.c0, s.dMom, nmMax, s.dDesc, enPolyW(P),
                          s.SZ, s.dPoly);
-      const long long nP = (long long)s.nClus * s.SZ;
-      if (nP > 0)
-        hipLaunchKernelGGL(k_to_f32, dim3((unsigned)((nP + 255) / 256)), dim3(256), 0, strm, s.dPoly, s.dPoly32,
-                           nP);
-    }
     if (hipGetLastError() != hipSuccess) { setErr("charge moment kernels failed"); return 0; }
     s.momReady = true;
+    s.polyReady32 = false;
+  }
+  if (f32 && s.uni && mode == 0 && !s.polyReady32) {   // the V table and the FP32 copy
+    const int nW = enPolyW(P);
+    hipLaunchKernelGGL(k_ct_poly, dim3(s.nClus), dim3(256), 0, strm, s.c0, s.dMom, nmMax, s.dDesc + nW, s.nDesc - nW,
+                       s.SZ, s.dPoly);
+    const long long nP = (long long)s.nClus * s.SZ;
+    if (nP > 0)
+      hipLaunchKernelGGL(k_to_f32, dim3((unsigned)((nP + 255) / 256)), dim3(256), 0, strm, s.dPoly, s.dPoly32, nP);
+    if (hipGetLastError() != hipSuccess) { setErr("charge moment kernels failed"); return 0; }
+    s.polyReady32 = true;
   }
   if (s.uni) {
     const int blocks = ((c->n + 64 * EN_WPB - 1) / (64 * EN_WPB)) * S;

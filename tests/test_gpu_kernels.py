@@ -63,3 +63,24 @@ def test_far_chain_orders(fa, tmp_path_factory, order, depth, mac):
     at = torch.empty_like(yd)
     op.matvec_t_dev(yd, at)
     assert abs(float(at.cpu().numpy() @ x) - float(y @ ax)) <= 1e-13 * np.linalg.norm(ax) * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("order,mac", [(1, 0.8), (2, 0.8), (5, 0.8), (6, 0.8), (7, 0.8), (8, 0.7), (9, 0.8)])
+def test_charge_walks_orders(fa, tmp_path_factory, order, mac):
+    """The walks' far term from one table per cluster (value and derivative along the normal
+    by one Horner scheme): energy, its weights' kappa derivative and the right-hand side."""
+    import torch
+    mesh = molecule(fa, tmp_path_factory, "globule", 3, 12, "--charges", "inside", "--nq", "400", "--sigma", "0.4",
+                    "--depth", "1.5", "--seed", "5")
+    tree = fa.Tree(mesh, 3, order=order, sep=mac)
+    ct = tree.charge_tree()
+    op = fa.Operator(tree, 0.1257, 1.0, 80.0, 1)
+    ora = O.Oracle(tree.oracle_layout(0.1257, 1.0, 80.0, 1))
+    op.set_charges(ct, mesh.pos, mesh.chr)
+    b = torch.empty(2 * tree.n, dtype=torch.float64, device="cuda")
+    op.rhs_tree_res_dev(b)
+    assert rel(b.cpu().numpy(), ora.rhs_tree(ct, mesh.pos, mesh.chr)) <= 1e-13
+    e = op.energy_res_dev(b)   # a density that does not cancel
+    assert abs(e - ora.energy(ct, mesh.pos, mesh.chr, b.cpu().numpy())) <= 1e-12 * abs(e)
+    assert abs(op.energy_res_dev(b, precision="fp32") - e) <= 3e-7 * abs(e)   # its tables built after the FP64 walk's
+    assert op.energy_res_dev(b) == e
