@@ -691,7 +691,7 @@ __global__ __launch_bounds__(256) void k_near_apply(const int2 *__restrict__ til
 // pairs.  Same tiles as k_near_apply.  The values differ from the stored
 // coefficients only by the rounding of the formula's operation order.
 #define FLY64_CHUNK 512   // staged source columns per pass
-#define FLY64_TAB 1024    // LDS entries of e^{-kappa r} at equal steps of r (NearK)
+#define FLY64_TAB 1536    // most LDS entries of e^{-kappa r} at equal steps of r (NearK)
 // 1/sqrt(x) for x > 0 (a normal FP64 number): the hardware estimate (relative
 // error 2^-24 measured on gfx950), then one third-order step
 // y <- y (1 + e/2 + 3e^2/8), e = 1 - x y^2, which cubes the error (measured
@@ -920,8 +920,8 @@ __device__ __forceinline__ void nearFly64Tile(const NearTile &tl, const int *__r
 // and has a block of its own: the launch of the default configuration, which
 // needs the registers of the mixed form's other branch (171 against 151 VGPRs)
 // for its third wave per SIMD.  Tiles costliest first (desc).
-// TAB: e^{-kappa r} from NearK's table (tab, K.nT entries), else from 2^(j/256)
-// and expNeg.  tr: the transposed operator's rows.
+// TAB: e^{-kappa r} from NearK's table (tab, K.nT entries in dynamic LDS), else from
+// 2^(j/256) (256 entries) and expNeg.  tr: the transposed operator's rows.
 #define MIX64_LDS (2 * NEAR_CHUNK * 8)
 #define FLY64_LDS (FLY64_CHUNK * (32 + 16 + 8 + 4))
 static_assert(MIX64_LDS >= FLY64_LDS, "the computed tiles' LDS must fit the union");
@@ -934,7 +934,7 @@ __global__ __launch_bounds__(256, 3) void k_near_mix64(
     const long long *__restrict__ specOff, const int *__restrict__ specCol, const double4 *__restrict__ specVal,
     double *__restrict__ out, int n, NearK K, const double *__restrict__ tab, int tr, int nTiles) {
   __shared__ __align__(16) unsigned char lds[MIX ? MIX64_LDS : FLY64_LDS];
-  __shared__ double sE[TAB ? FLY64_TAB : 256];
+  double *sE = reinterpret_cast<double *>(dynLds);
   for (int j = threadIdx.x; j < (TAB ? K.nT : 256); j += blockDim.x) sE[j] = TAB ? tab[j] : gExp2Tab[j];
   double4 *sP = reinterpret_cast<double4 *>(lds);
   double2 *sM = reinterpret_cast<double2 *>(sP + FLY64_CHUNK);
@@ -5917,10 +5917,14 @@ static void farPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_t
 
 // The FP64 mixed nearfield of the operator (tr 0) or its transpose into c->nearv.
 // e^{-kappa r} comes from the table of steps wherever the near distances fit its
-// FLY64_TAB entries (kappa r up to 4: every leaf size in use); beyond it expNeg.
+// FLY64_TAB entries: kappa r up to 6, the near lists of a capsid wall's leaves among
+// them (they reach 4.1; with the line at 4 the matvec of 655k panels took 5,328 us by
+// expNeg, 5,218 by the table); beyond it expNeg.  A block holds only the entries in use
+// (346 at 317k panels), so that the longest table does not cost the others LDS.
+static size_t nearTabLds(const NearK &K) { return (K.nT > 0 ? K.nT : 256) * sizeof(double); }
 static void nearMix64(fbh_ctx *c, const double4 *coef, const double4 *spec, const double *x, int tr, hipStream_t st) {
   auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(c->nearGrid), dim3(256), 0, st, c->nearDesc, c->tiles, c->leafStart, c->leafCount,
+    hipLaunchKernelGGL(kern, dim3(c->nearGrid), dim3(256), nearTabLds(c->nearK[tr]), st, c->nearDesc, c->tiles, c->leafStart, c->leafCount,
                        c->srcOff, c->ncol, c->tileCoef, c->srcList, coef, c->fly64PA, c->fly64PN, x, c->specOff,
                        c->specCol, spec, c->nearv, c->n, c->nearK[tr], c->nearTab, tr, c->nTiles);
   };
