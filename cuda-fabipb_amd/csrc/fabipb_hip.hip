@@ -2713,39 +2713,45 @@ __global__ __launch_bounds__(256) void k_rhs(const Pnl *__restrict__ pnl, int n,
 
 #pragma clang fp contract(fast)
 // the direct right-hand side at q = 1: one quadrature point per panel, so the
-// point and its weight 2 A t w w leave the charge loop; 1/r from rsqrt
-__global__ __launch_bounds__(256) void k_rhs_q1(const Pnl *__restrict__ pnl, int n, int nChar,
-                                                const double *__restrict__ pos, const double *__restrict__ chr,
-                                                double *__restrict__ b, double fac, double t, double ww) {
-  __shared__ double4 sp[256];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double xq[3] = {0, 0, 0}, nr[3] = {0, 0, 0}, W = 0.0;
-  if (i < n) {
-    const Pnl &P = pnl[i];
-    for (int k = 0; k < 3; k++) {
-      xq[k] = P.v[k] + t * (P.a[6 + k] + t * P.a[k]);
-      nr[k] = P.nr[k];
-    }
-    W = ww * 2.0 * P.area * fac;
+// point and its weight 2 A t w w leave the charge loop; 1/r from rsqrt.  FP64
+// issue bounds it where enough waves run: a block takes 64 panels and its
+// blockDim / 64 waves share the charges (a contiguous range each, read as scalars;
+// their sums are added in wave order), where one lane per panel over all charges
+// left five waves on a CU and, at 81,920 panels, a quarter of the CUs with twice the
+// work.  2,000 charges: 210 -> 137 us; 5,120 panels, 200 charges: 15.6 -> 7.0.
+#define RHS_WAVES 16   // most waves a block
+__global__ __launch_bounds__(64 * RHS_WAVES) void k_rhs_q1(const Pnl *__restrict__ pnl, int n, int nChar,
+                                                           const double *__restrict__ pos,
+                                                           const double *__restrict__ chr, double *__restrict__ b,
+                                                           double fac, double t, double ww) {
+  __shared__ double red[2][RHS_WAVES][64];
+  const int nw = blockDim.x >> 6, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 64 + lane;
+  const Pnl &P = pnl[min(i, n - 1)];
+  double xq[3], nr[3];
+  for (int k = 0; k < 3; k++) {
+    xq[k] = P.v[k] + t * (P.a[6 + k] + t * P.a[k]);
+    nr[k] = P.nr[k];
   }
+  const double W = ww * 2.0 * P.area * fac;
+  const int per = (nChar + nw - 1) / nw, j1 = min(nChar, (w + 1) * per);
   double b0 = 0.0, b1 = 0.0;
-  for (int j0 = 0; j0 < nChar; j0 += 256) {
-    __syncthreads();
-    const int j = j0 + threadIdx.x;
-    if (j < nChar) sp[threadIdx.x] = make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], chr[j]);
-    __syncthreads();
-    const int cnt = min(256, nChar - j0);
 #pragma unroll 4
-    for (int jj = 0; jj < cnt; jj++) {
-      const double4 c = sp[jj];
-      const double rx = xq[0] - c.x, ry = xq[1] - c.y, rz = xq[2] - c.z;
-      const double r2 = rx * rx + ry * ry + rz * rz, ri = rsqrt(r2);
-      const double ip = nr[0] * rx + nr[1] * ry + nr[2] * rz;
-      b0 += c.w * ri;
-      b1 -= c.w * ip * (ri * ri * ri);
-    }
+  for (int j = w * per; j < j1; j++) {
+    const double rx = xq[0] - pos[3 * j], ry = xq[1] - pos[3 * j + 1], rz = xq[2] - pos[3 * j + 2], c = chr[j];
+    const double r2 = rx * rx + ry * ry + rz * rz, ri = rsqrt(r2);
+    const double ip = nr[0] * rx + nr[1] * ry + nr[2] * rz;
+    b0 += c * ri;
+    b1 -= c * ip * (ri * ri * ri);
   }
-  if (i < n) {
+  red[0][w][lane] = b0;
+  red[1][w][lane] = b1;
+  __syncthreads();
+  if (w == 0 && i < n) {
+    for (int k = 1; k < nw; k++) {
+      b0 += red[0][k][lane];
+      b1 += red[1][k][lane];
+    }
     b[i] = b0 * W;
     b[i + n] = b1 * W;
   }
@@ -2931,17 +2937,24 @@ __global__ __launch_bounds__(256) void k_grad_q(const Pnl *__restrict__ pnl, int
 
 // (R^T lam)_j at q = 1 (the transposed k_rhs_q1): block (charge tile, panel
 // chunk); each panel's point, normal and two weights fac 2A t w w (lam,
-// lam_n) staged once per chunk; 1/r from rsqrt; part[chunk][j] as k_grad_q
+// lam_n) staged once per chunk; 1/r from rsqrt; part[chunk][j] as k_grad_q.
+// A lane takes two charges, so that a staged panel's 64 bytes of LDS serve two
+// pairs (one charge a lane: LDS reads bound it), and the four waves a quarter of the
+// staged panels each, which keeps the tiles small; their sums are added in wave
+// order.  82k panels, 5,000 charges: 441 -> 371 us.
+#define GRADR_TILE 128
 __global__ __launch_bounds__(256) void k_gradR_q1(const Pnl *__restrict__ pnl, int n, int nChar,
                                                   const double *__restrict__ pos, const double *__restrict__ lam,
                                                   double *__restrict__ part, double fac, double t, double ww) {
   __shared__ double4 sp[256], sn[256];   // (point, fac W lam), (normal, fac W lam_n)
-  const int j = blockIdx.x * 256 + threadIdx.x;
+  __shared__ double red[4][GRADR_TILE];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int t0 = blockIdx.x * GRADR_TILE;
   const int p0 = blockIdx.y * GRAD_PCH, p1 = min(n, p0 + GRAD_PCH);
-  double c[3] = {0, 0, 0};
-  if (j < nChar)
-    for (int k = 0; k < 3; k++) c[k] = pos[3 * j + k];
-  double acc = 0.0;
+  double c[2][3], acc[2] = {0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 2; q++)
+    for (int k = 0; k < 3; k++) c[q][k] = pos[3 * min(t0 + lane + 64 * q, nChar - 1) + k];
   for (int b0 = p0; b0 < p1; b0 += 256) {
     __syncthreads();
     const int pi = b0 + threadIdx.x;
@@ -2955,16 +2968,24 @@ __global__ __launch_bounds__(256) void k_gradR_q1(const Pnl *__restrict__ pnl, i
     }
     __syncthreads();
     const int cnt = min(256, p1 - b0);
-#pragma unroll 4
-    for (int jj = 0; jj < cnt; jj++) {
+#pragma unroll 2
+    for (int jj = w; jj < cnt; jj += 4) {
       const double4 a = sp[jj], m = sn[jj];
-      const double rx = a.x - c[0], ry = a.y - c[1], rz = a.z - c[2];
-      const double r2 = rx * rx + ry * ry + rz * rz, ri = rsqrt(r2);
-      const double ip = m.x * rx + m.y * ry + m.z * rz;
-      acc += a.w * ri - m.w * ip * (ri * ri * ri);
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const double rx = a.x - c[q][0], ry = a.y - c[q][1], rz = a.z - c[q][2];
+        const double r2 = rx * rx + ry * ry + rz * rz, ri = rsqrt(r2);
+        const double ip = m.x * rx + m.y * ry + m.z * rz;
+        acc[q] += a.w * ri - m.w * ip * (ri * ri * ri);
+      }
     }
   }
-  if (j < nChar) part[(long long)blockIdx.y * nChar + j] = acc;
+  red[w][lane] = acc[0];
+  red[w][lane + 64] = acc[1];
+  __syncthreads();
+  const int k = threadIdx.x;
+  if (k < GRADR_TILE && t0 + k < nChar)
+    part[(long long)blockIdx.y * nChar + t0 + k] = ((red[0][k] + red[1][k]) + red[2][k]) + red[3][k];
 }
 
 __global__ void k_grad_sum(const double *__restrict__ part, int nChunk, int nChar, double *__restrict__ out,
@@ -7040,10 +7061,15 @@ static int rhsDirect(fbh_ctx *c, int nChar, const double *dp, const double *dc, 
   if (fp32 && c->qorder == 1)
     hipLaunchKernelGGL(k_rhs32_q1, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->pnl, c->n, nChar, dp, dc,
                        b_dev, fac, c->Q.t[0], c->Q.t[0] * c->Q.w[0] * c->Q.w[0]);
-  else if (c->qorder == 1)
-    hipLaunchKernelGGL(k_rhs_q1, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->pnl, c->n, nChar, dp, dc,
-                       b_dev, fac, c->Q.t[0], c->Q.t[0] * c->Q.w[0] * c->Q.w[0]);
-  else
+  else if (c->qorder == 1) {
+    // four waves a block (five a SIMD at 82k panels), more while the panels alone
+    // leave fewer than that and each wave keeps eight charges
+    const int blocks = (c->n + 63) / 64;
+    int nw = 4;
+    while (nw < RHS_WAVES && blocks * nw < 20 * 256 && nChar >= 16 * nw) nw *= 2;
+    hipLaunchKernelGGL(k_rhs_q1, dim3(blocks), dim3(64 * nw), 0, c->stream, c->pnl, c->n, nChar, dp, dc, b_dev, fac,
+                       c->Q.t[0], c->Q.t[0] * c->Q.w[0] * c->Q.w[0]);
+  } else
     hipLaunchKernelGGL(k_rhs, dim3((c->n + 255) / 256), dim3(256), 0, c->stream, c->pnl, c->n, nChar, dp, dc, b_dev,
                        fac, c->Q, c->qorder);
   hipError_t e = hipGetLastError();
@@ -7811,8 +7837,8 @@ extern "C" int fbh_gradient_tree_dev(fbh_ctx *c, int nChar, const double *pos, c
   if (!adjEval(c, s, lamBuf, phi, dq)) return 0;
   if (!rhsTree) {   // R^T lam by the direct sums
     if (c->qorder == 1)
-      hipLaunchKernelGGL(k_gradR_q1, dim3((nChar + 255) / 256, nChunk), dim3(256), 0, c->stream, c->pnl, n, nChar,
-                         s.dPos, lam_dev, part, rhsFactor(c), c->Q.t[0], c->Q.t[0] * c->Q.w[0] * c->Q.w[0]);
+      hipLaunchKernelGGL(k_gradR_q1, dim3((nChar + GRADR_TILE - 1) / GRADR_TILE, nChunk), dim3(256), 0, c->stream,
+                         c->pnl, n, nChar, s.dPos, lam_dev, part, rhsFactor(c), c->Q.t[0], c->Q.t[0] * c->Q.w[0] * c->Q.w[0]);
     else
       hipLaunchKernelGGL(k_grad_q<false>, dim3((nChar + 255) / 256, nChunk), dim3(256), 0, c->stream, c->pnl, n,
                          nChar, s.dPos, (const double *)nullptr, lam_dev, part, c->kappa, c->eps, rhsFactor(c), c->Q,

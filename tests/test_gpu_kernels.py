@@ -84,3 +84,43 @@ def test_charge_walks_orders(fa, tmp_path_factory, order, mac):
     assert abs(e - ora.energy(ct, mesh.pos, mesh.chr, b.cpu().numpy())) <= 1e-12 * abs(e)
     assert abs(op.energy_res_dev(b, precision="fp32") - e) <= 3e-7 * abs(e)   # its tables built after the FP64 walk's
     assert op.energy_res_dev(b) == e
+
+
+@pytest.mark.parametrize("nchar", [1, 15, 33, 127, 130, 1000])
+def test_direct_charge_sums(fa, tmp_path_factory, nchar):
+    """The direct right-hand side (its charges split over the waves of a block) and its
+    transpose (tiles of 128 charges), for counts around the splits; 1,272 panels, the last
+    block of 64 partly empty.  2e-14: 2,000 roundings of 2^-53 against the largest sum."""
+    import torch
+    mesh = molecule(fa, tmp_path_factory, "globule", 3, 8, *GLOBULE)
+    tree = fa.Tree(mesh, 2, order=6)
+    rng = np.random.default_rng(nchar)
+    pos = rng.uniform(-2, 2, (nchar, 3))
+    q = rng.normal(0, 0.4, nchar)
+    op = fa.Operator(tree, 0.1257, 1.0, 80.0, 1)
+    ora = O.Oracle(tree.oracle_layout(0.1257, 1.0, 80.0, 1))
+    b = op.rhs(pos, q)
+    ref = ora.rhs(pos, q)
+    one = [ora.rhs(pos[k:k + 1], np.abs(q[k:k + 1])) for k in range(min(nchar, 4))]
+    scale = np.abs(ref).max() + sum(np.abs(o).max() for o in one)
+    assert np.abs(b - ref).max() <= 2e-14 * scale
+
+
+@pytest.mark.parametrize("nchar", [7, 127, 130, 400])
+def test_direct_gradient_sums(fa, tmp_path_factory, nchar):
+    """R^T lam by tiles of 128 charges (the transposed direct right-hand side): the gradient
+    of a zero density, against the oracle's right-hand sides of unit charges; counts around
+    the tile.  1,278 panels: 3e-13 covers the roundings of 2,556 terms of 2^-53 each."""
+    import torch
+    mesh = molecule(fa, tmp_path_factory, "globule", 3, 12, "--charges", "inside", "--nq", str(nchar), "--sigma", "0.4",
+                    "--depth", "1.5", "--seed", "5", "--merge", "0.6")
+    tree = fa.Tree(mesh, 2, order=6)
+    op = fa.Operator(tree, 0.1257, 1.0, 80.0, 1)
+    ora = O.Oracle(tree.oracle_layout(0.1257, 1.0, 80.0, 1))
+    lam = torch.tensor(np.random.default_rng(3).uniform(-1, 1, 2 * tree.n), device="cuda")
+    dq, _, _ = op.gradient_tree_dev(tree.charge_tree(), mesh.pos, mesh.chr, torch.zeros_like(lam), lam, tol=1e-8)
+    u = lam.cpu().numpy()
+    cols = [ora.rhs(mesh.pos[k:k + 1], np.ones(1)) for k in range(nchar)]
+    want = np.array([u @ c for c in cols])
+    tot = np.array([np.abs(u) @ np.abs(c) for c in cols])
+    assert (np.abs(dq - want) <= 3e-13 * tot).all()
