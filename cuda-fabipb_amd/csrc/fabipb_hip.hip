@@ -2436,6 +2436,12 @@ __global__ __launch_bounds__(256) void k_l2lp(const R *__restrict__ Q0, const R 
   }
 }
 
+// y = alpha*(D x - far - near) + beta*y where the L2P ends the product (k_combine)
+struct Combine {
+  const double *x, *nearv, *area;
+  double *y, alpha, beta, s1, s2;   // y null: the far part alone, into far
+};
+
 // The FP64 downward pass of one leaf: L2L down its ancestry and L2P as k_l2lp,
 // on the two sums the panels need (u = l1 + l2 against the moments, v = l3 + l4
 // against the noments; translation is linear, so they are formed before it) and
@@ -2454,7 +2460,7 @@ __global__ __launch_bounds__(256) void k_l2lp64(const double *__restrict__ Q0, c
                                                 const int *__restrict__ anc, LevOrd O,
                                                 const double *__restrict__ cubeX, const double *__restrict__ lec,
                                                 double *__restrict__ far, int n, int nm, int nmMax, int nUp, int nAnc,
-                                                DevTabs T) {
+                                                DevTabs T, Combine C) {
   typedef double VT __attribute__((ext_vector_type(V)));
   __shared__ double co[L2LP_MAXUP][3][MAXP + 1];   // t_d^k / k! of each step
   __shared__ double4 wt[256];                      // the panels' normals
@@ -2564,7 +2570,15 @@ __global__ __launch_bounds__(256) void k_l2lp64(const double *__restrict__ Q0, c
       if (j0 + 16 < cn) fetch(j0 + 16);   // in flight under the reduction
       const double r = waveSum8(v8, lane);
       const int k = lane >> 4, which = (lane >> 3) & 1;
-      if ((lane & 7) == 0 && j0 + k < cn) far[s0 + c0 + j0 + k + (which != (TR ? 1 : 0) ? n : 0)] = r;
+      if ((lane & 7) == 0 && j0 + k < cn) {
+        const int p = s0 + c0 + j0 + k, i = p + (which != (TR ? 1 : 0) ? n : 0);
+        if (C.y) {
+          const double v = C.alpha * ((i < n ? C.s1 : C.s2) * C.area[p] * C.x[i] - (r + C.nearv[i]));
+          C.y[i] = C.beta == 0.0 ? v : v + C.beta * C.y[i];
+        } else {
+          far[i] = r;
+        }
+      }
     }
   }
 }
@@ -5856,14 +5870,14 @@ static void q2m64(const fbh_ctx *c, const double *x, double *mom, int swap, hipS
 }
 // nUp: levels translated down before the L2P (0: from the leaves' own locals)
 template <bool TR>
-static void l2lp64(const fbh_ctx *c, const double *lec, double *far, int nUp, hipStream_t st) {
+static void l2lp64(const fbh_ctx *c, const double *lec, double *far, int nUp, hipStream_t st, const Combine &C = {}) {
   LevOrd O{};
   for (int s = 0; s <= nUp; s++) O.p[s] = c->ordMom[c->depth - nUp + s];
   const size_t lds = (size_t)(nUp + 2) * c->nmMax * sizeof(double2);
   withSlots(c->nmLeaf, [&](auto V, auto NL) {
     hipLaunchKernelGGL((k_l2lp64<V.value, NL.value, TR>), dim3(c->nLeaf), dim3(256), lds, st, c->Q0, c->fly64PN,
                        c->leafStart, c->leafCount, c->leafAnc, O, c->cubeX, lec, far, c->n, c->nmLeaf, c->nmMax, nUp,
-                       c->depth - c->height + 1, c->T);
+                       c->depth - c->height + 1, c->T, C);
   });
 }
 
@@ -5911,10 +5925,10 @@ static bool l2lpFits(const fbh_ctx *c) {
   return l2lpLds<R>(c) <= (size_t)c->ldsMax && c->depth - c->height <= L2LP_MAXUP;
 }
 template <typename R>
-static bool l2lpPass(fbh_ctx *c, const OpBufs<R> &B, hipStream_t st) {
+static bool l2lpPass(fbh_ctx *c, const OpBufs<R> &B, hipStream_t st, const Combine &C = {}) {
   if (!l2lpFits<R>(c)) return false;
   if constexpr (std::is_same<R, double>::value) {
-    l2lp64<false>(c, B.lec, B.far, c->depth - c->height, st);
+    l2lp64<false>(c, B.lec, B.far, c->depth - c->height, st, C);
   } else {
     const int V = vecWidth<R>(c->nmLeaf), nmx = c->nmMax, nUp = c->depth - c->height;
     const size_t lds = l2lpLds<R>(c);
@@ -5950,14 +5964,16 @@ static bool m2mAxPass(fbh_ctx *c, const OpBufs<R> &B, int lev, hipStream_t st) {
 
 // far field into B.far: Q2M, M2M (finest parent level up), M2L, L2L (down), L2P.
 // staged: L2L level by level into B.lec and a separate L2P (the stage ABI reads
-// the locals of every cube afterwards); else L2L and L2P in one launch.
+// the locals of every cube afterwards); else L2L and L2P in one launch, which ends
+// the product where C has a y (only where l2lpFits).
 template <typename R>
-static void farPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_t st, bool staged = false) {
+static void farPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_t st, bool staged = false,
+                    const Combine &C = {}) {
   q2mPass(c, B, x, st);
   for (int lev = c->depth - 1; lev >= c->height; lev--)
     if (staged || !m2mAxPass(c, B, lev, st)) m2mPass(c, B, lev, st);
   m2lPass(c, B, st);
-  if (!staged && l2lpPass(c, B, st)) return;
+  if (!staged && l2lpPass(c, B, st, C)) return;
   for (int lev = c->height; lev < c->depth; lev++) l2lPass(c, B, lev, st);
   l2pPass(c, B, st);
 }
@@ -6007,6 +6023,20 @@ static void directPass(fbh_ctx *c, const double *x, double *out, hipStream_t st)
                      c->dSrcOff, c->dNcol, c->dTileCoef, c->dSrcList, c->dCoef, x, out, c->n);
 }
 
+// Small products run as one chain of launches on one stream, the nearfield first and
+// the combine inside the L2P: two events, two waits and a launch less, against an
+// overlap worth at most the nearfield's time.  1,280 panels: 74 us on two streams,
+// 57 so; solves of 5,120 panels: 2.0M near pairs 1,121 -> 947 us, 7.3M 1,130 ->
+// 1,034; 20,480 panels, 26M: 2,370 -> 2,450.  Streamed pairs (q > 1) take three
+// times as long as computed ones.
+#define ONE_STREAM_PAIRS 10000000LL
+static bool oneStream(const fbh_ctx *c) {
+  return c->nInter * (c->qorder > 1 ? 3 : 1) <= ONE_STREAM_PAIRS && l2lpFits<double>(c);
+}
+static Combine combineOf(const fbh_ctx *c, double alpha, const double *x, double beta, double *y) {
+  return {x, c->nearv, c->area, y, alpha, beta, (1.0 + c->eps) / 2.0, (1.0 + 1.0 / c->eps) / 2.0};
+}
+
 // y = alpha*(D - K) x + beta*y; the nearfield runs on the side stream beside
 // the far-field chain (both read x only) and the combine waits for both
 template <typename R>
@@ -6021,15 +6051,25 @@ static int matvecT(fbh_ctx *c, const OpBufs<R> &B, double alpha, const double *x
     HCK(hipGetLastError());
     return 1;
   }
-  HCK(hipEventRecord(c->evFork, c->stream));
-  hipStream_t ns = c->side;
-  HCK(hipStreamWaitEvent(ns, c->evFork, 0));
+  bool one = false;
+  if constexpr (std::is_same<R, double>::value) one = oneStream(c);
+  hipStream_t ns = one ? c->stream : c->side;
+  if (!one) {
+    HCK(hipEventRecord(c->evFork, c->stream));
+    HCK(hipStreamWaitEvent(ns, c->evFork, 0));
+  }
   const bool timed = c->ntOn && 2 * (size_t)c->ntUsed + 1 < c->ntEv.size();
   if (timed) HCK(hipEventRecord(c->ntEv[2 * c->ntUsed], ns));
   nearPass(c, B, x, ns);
   if (timed) {
     HCK(hipEventRecord(c->ntEv[2 * c->ntUsed + 1], ns));
     c->ntKind[c->ntUsed++] = sizeof(R) == 4;
+  }
+  if (one) {
+    if constexpr (std::is_same<R, double>::value)
+      farPass(c, B, x, c->stream, false, combineOf(c, alpha, x, beta, y));
+    HCK(hipGetLastError());
+    return 1;
   }
   HCK(hipEventRecord(c->evJoin, ns));
   farPass(c, B, x, c->stream);
@@ -6082,8 +6122,9 @@ static int ensureAdjoint(fbh_ctx *c) {
   return 1;
 }
 
-// the transposed far chain from y into c->far (adjL: adjoint locals, adjM: adjoint moments)
-static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
+// the transposed far chain from y into c->far (adjL: adjoint locals, adjM: adjoint moments);
+// C as in farPass
+static void farPassT(fbh_ctx *c, const double *y, hipStream_t st, const Combine &C = {}) {
   q2m64(c, y, c->adjL, 1, st);
   OpBufs<double> B = bufs64(c);
   B.mom = c->adjL;
@@ -6099,7 +6140,7 @@ static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
   else if (c->m2lMaxT == 32) launch(k_m2l_cached<double, 32, true>);
   else launch(k_m2l_cached<double, 0, true>);
   if (l2lpFits<double>(c)) {
-    l2lp64<true>(c, c->adjM, c->far, c->depth - c->height, st);
+    l2lp64<true>(c, c->adjM, c->far, c->depth - c->height, st, C);
     return;
   }
   for (int lev = c->height; lev < c->depth; lev++) {
@@ -6117,14 +6158,23 @@ static void farPassT(fbh_ctx *c, const double *y, hipStream_t st) {
 static int matvecTr(fbh_ctx *c, double alpha, const double *x, double beta, double *y) {
   if (c->direct) { setErr("the adjoint operator has no direct (-r) form"); return 0; }
   if (!ensureAdjoint(c)) return 0;
-  HCK(hipEventRecord(c->evFork, c->stream));
-  HCK(hipStreamWaitEvent(c->side, c->evFork, 0));
+  const bool one = oneStream(c);
+  hipStream_t ns = one ? c->stream : c->side;
+  if (!one) {
+    HCK(hipEventRecord(c->evFork, c->stream));
+    HCK(hipStreamWaitEvent(ns, c->evFork, 0));
+  }
   if (c->nFlyTiles > 0)
-    nearMix64(c, c->coefT, c->specValT64, x, 1, c->side);
+    nearMix64(c, c->coefT, c->specValT64, x, 1, ns);
   else
-    hipLaunchKernelGGL(k_near_apply<double>, dim3(c->nTiles), dim3(256), 0, c->side, c->tiles, c->leafStart,
+    hipLaunchKernelGGL(k_near_apply<double>, dim3(c->nTiles), dim3(256), 0, ns, c->tiles, c->leafStart,
                        c->leafCount, c->srcOff, c->ncol, c->tileCoef, c->srcList, c->coefT, x, c->nearv, c->n);
-  HCK(hipEventRecord(c->evJoin, c->side));
+  if (one) {
+    farPassT(c, x, c->stream, combineOf(c, alpha, x, beta, y));
+    HCK(hipGetLastError());
+    return 1;
+  }
+  HCK(hipEventRecord(c->evJoin, ns));
   farPassT(c, x, c->stream);
   HCK(hipStreamWaitEvent(c->stream, c->evJoin, 0));
   const double s1 = (1.0 + c->eps) / 2.0, s2 = (1.0 + 1.0 / c->eps) / 2.0;

@@ -124,3 +124,28 @@ def test_direct_gradient_sums(fa, tmp_path_factory, nchar):
     want = np.array([u @ c for c in cols])
     tot = np.array([np.abs(u) @ np.abs(c) for c in cols])
     assert (np.abs(dq - want) <= 3e-13 * tot).all()
+
+
+@pytest.mark.parametrize("depth", [2, 4])
+def test_product_in_place(fa, tmp_path_factory, depth):
+    """The product whose combine ends the L2P (up to 10M near pairs; depth 2 of 20,480 panels is
+    above it, depth 4 below): alpha, beta and y = x, forward and transposed, against the
+    oracle and against the two-argument form."""
+    import torch
+    mesh = molecule(fa, tmp_path_factory, "sphere", 5, 20, "--charges", "ball", "--nq", "20", "--rq", "12", "--seed", "3")
+    tree = fa.Tree(mesh, depth, order=6)
+    op = fa.Operator(tree, 0.1257, 1.0, 80.0, 1)
+    assert (op.stats()["near_interactions"] > 10_000_000) == (depth == 2)
+    x, y0 = np.random.default_rng(4).uniform(-1, 1, (2, 2 * tree.n))
+    ora = O.Oracle(tree.oracle_layout(0.1257, 1.0, 80.0, 1))
+    ax = ora.matvec(x)
+    assert rel(op.matvec(x, 0.75, -0.5, y0.copy()), 0.75 * ax - 0.5 * y0) <= 1e-13
+    xd = torch.tensor(x, device="cuda")
+    for f in (op.matvec_dev, op.matvec_t_dev):
+        y, z = torch.tensor(y0, device="cuda"), xd.clone()
+        f(xd, y, alpha=0.75, beta=-0.5)
+        f(z, z)
+        p = torch.empty_like(xd)
+        f(xd, p)
+        assert torch.equal(z, p)
+        assert rel(y.cpu().numpy(), 0.75 * p.cpu().numpy() - 0.5 * y0) <= 1e-14
