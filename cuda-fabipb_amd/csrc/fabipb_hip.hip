@@ -4544,20 +4544,24 @@ __global__ __launch_bounds__(256) void k_mgs_dot(double *__restrict__ w, const d
   if (threadIdx.x == 0) partOut[blockIdx.x] = s[0];
 }
 
-// h = ||w||; v = w / h if h > 0 (src/gmres.c:612-620)
+// h[i] = ||w||; v = w / h[i] if h[i] > 0 (src/gmres.c:612-620).  Block 0 also stores
+// the finished Hessenberg column h[0..i] to pinned host memory, which the host reads
+// after the launch: a copy command of its own cost 2.5 us and its gap per Arnoldi step.
 __global__ __launch_bounds__(256) void k_normalize(const double *__restrict__ w, double *__restrict__ v, int n,
-                                                   const double *__restrict__ part, double *__restrict__ h) {
+                                                   const double *__restrict__ part, const double *__restrict__ h,
+                                                   int i, double *__restrict__ hostH) {
   double hh = sqrt(reduceParts(part, RED_BLOCKS));
-  if (blockIdx.x == 0 && threadIdx.x == 0) *h = hh;
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k <= i; k += 256) hostH[k] = k < i ? h[k] : hh;
   double sc = hh > 0.0 ? 1.0 / hh : 1.0;
   const int st = gridDim.x * 256;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += RED_U * st) {
+  for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += RED_U * st) {
     double wv[RED_U];
 #pragma unroll
-    for (int u = 0; u < RED_U; u++) wv[u] = i + u * st < n ? w[i + u * st] : 0.0;
+    for (int u = 0; u < RED_U; u++) wv[u] = j + u * st < n ? w[j + u * st] : 0.0;
 #pragma unroll
     for (int u = 0; u < RED_U; u++)
-      if (i + u * st < n) v[i + u * st] = hh > 0.0 ? wv[u] * sc : wv[u];
+      if (j + u * st < n) v[j + u * st] = hh > 0.0 ? wv[u] * sc : wv[u];
   }
 }
 
@@ -6737,14 +6741,14 @@ static int streamSpin(fbh_ctx *c) {
 }
 
 // 2-norms of k <= 4 device vectors of 2n: k deterministic reductions (as
-// k_dot_part + k_sum_parts do for one), one pinned readback, one wait
+// k_dot_part + k_sum_parts do for one), each stored to pinned host memory, one wait
 static int devNorms(fbh_ctx *c, int k, const double *const *v, double *out) {
   const int n2 = 2 * c->n;
   for (int q = 0; q < k; q++) {
     hipLaunchKernelGGL(k_dot_part, dim3(RED_BLOCKS), dim3(256), 0, c->stream, v[q], v[q], n2, c->part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, c->stream, c->part, RED_BLOCKS, c->scal + q);
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, c->stream, c->part, RED_BLOCKS, c->hpin + q);
   }
-  HCK(hipMemcpyAsync(c->hpin, c->scal, k * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HCK(hipGetLastError());
   if (!streamSpin(c)) return 0;
   for (int q = 0; q < k; q++) out[q] = sqrt(c->hpin[q]);
   return 1;
@@ -6858,9 +6862,9 @@ static int gmresCore(fbh_ctx *c, int kind, const double *b, double *x, int restr
                            c->hcol + k, pb);
         std::swap(pa, pb);
       }
-      hipLaunchKernelGGL(k_normalize, dim3(RED_BLOCKS), dim3(256), 0, c->stream, c->w, vn, n2, pa, c->hcol + i);
+      hipLaunchKernelGGL(k_normalize, dim3(RED_BLOCKS), dim3(256), 0, c->stream, c->w, vn, n2, pa, c->hcol, i,
+                         c->hpin);
       HCK(hipGetLastError());
-      HCK(hipMemcpyAsync(c->hpin, c->hcol, (i + 1) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
       if (!streamSpin(c)) return 0;
       double *h = &H[(size_t)(i - 1) * ldh];
       for (int k = 0; k <= i; k++) h[k] = c->hpin[k];
