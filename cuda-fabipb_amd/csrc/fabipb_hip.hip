@@ -6741,9 +6741,12 @@ extern "C" int fbh_psolve_dev(fbh_ctx *c, double *out, const double *in) {
     return 1;
   }
   if (c->precMode != 2) return fbh_psolve_diag_dev(c, out, in);
-  HCK(hipMemcpyAsync(c->pbTmp, in, 2 * (size_t)c->n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+  if (in < out + 2 * (size_t)c->n && out < in + 2 * (size_t)c->n) {   // a block's rows are written while others read its x
+    HCK(hipMemcpyAsync(c->pbTmp, in, 2 * (size_t)c->n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    in = c->pbTmp;
+  }
   hipLaunchKernelGGL(k_bp_apply, dim3(c->nPBTiles), dim3(256), 0, c->stream, c->pbTiles, c->pbStart, c->pbM, c->pbOff,
-                     c->pbInv, c->pbTmp, out, c->n);
+                     c->pbInv, in, out, c->n);
   HCK(hipGetLastError());
   return 1;
 }
@@ -6832,9 +6835,12 @@ static int precApply(fbh_ctx *c, int kind, double *out, const double *in) {
                        c->pbInvT);
     HCK(hipGetLastError());
   }
-  HCK(hipMemcpyAsync(c->pbTmp, in, 2 * (size_t)c->n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+  if (in < out + 2 * (size_t)c->n && out < in + 2 * (size_t)c->n) {
+    HCK(hipMemcpyAsync(c->pbTmp, in, 2 * (size_t)c->n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    in = c->pbTmp;
+  }
   hipLaunchKernelGGL(k_bp_apply, dim3(c->nPBTiles), dim3(256), 0, c->stream, c->pbTiles, c->pbStart, c->pbM, c->pbOff,
-                     c->pbInvT, c->pbTmp, out, c->n);
+                     c->pbInvT, in, out, c->n);
   HCK(hipGetLastError());
   return 1;
 }
@@ -6890,7 +6896,9 @@ static int gmresCore(fbh_ctx *c, int kind, const double *b, double *x, int restr
       ++i;
       ++*iters;
       double *vi = c->V + (size_t)(i - 1) * n2, *vn = c->V + (size_t)i * n2;
-      if (!applyOp(c, kind, 1.0, vi, 0.0, c->w)) return 0;
+      // the block preconditioner is not applied in place: the product goes to its buffer
+      double *av = c->precMode == 2 ? c->pbTmp : c->w;
+      if (!applyOp(c, kind, 1.0, vi, 0.0, av)) return 0;
       // modified Gram-Schmidt: <w, v0> (with the diagonal preconditioner applied
       // in the same pass), then per k the update fused with the next dot product
       double *pa = c->part, *pb = c->part + RED_BLOCKS;
@@ -6898,7 +6906,7 @@ static int gmresCore(fbh_ctx *c, int kind, const double *b, double *x, int restr
         hipLaunchKernelGGL(k_psolve_dot, dim3(RED_BLOCKS), dim3(256), 0, c->stream, c->w, c->V, c->area, c->n,
                            (1.0 + c->eps) / 2.0, (1.0 + 1.0 / c->eps) / 2.0, pa);
       } else {
-        if (!precApply(c, kind, c->w, c->w)) return 0;
+        if (!precApply(c, kind, c->w, av)) return 0;
         hipLaunchKernelGGL(k_dot_part, dim3(RED_BLOCKS), dim3(256), 0, c->stream, c->w, c->V, n2, pa);
       }
       for (int k = 0; k < i; k++) {
