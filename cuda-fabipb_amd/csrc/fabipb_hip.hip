@@ -3391,47 +3391,54 @@ __global__ void k_ct_leaf(int levStart, const int *__restrict__ chgStart, const 
 }
 
 // upward pass of the charge moments (src/chargeTree.c:344-395, transM2Mchr)
-__global__ void k_ct_m2m(int levStart, const int *__restrict__ kidStart, const int *__restrict__ nKids,
-                         const double *__restrict__ ctx_, const int *__restrict__ ordOf, int lev,
-                         double *__restrict__ cmom, int nmMax, DevTabs T) {
+// One wave per kid (at most eight), lanes over multi-indices, the kids' contributions
+// added in kid order: a kid's chain of dependent LDS reads is all a block waits for,
+// where one wave took the kids one after the other (5,000 charges, a level: 61 -> 12 us).
+__global__ __launch_bounds__(512) void k_ct_m2m(int levStart, const int *__restrict__ kidStart,
+                                                const int *__restrict__ nKids, const double *__restrict__ ctx_,
+                                                const int *__restrict__ ordOf, int lev, double *__restrict__ cmom,
+                                                int nmMax, DevTabs T) {
   extern __shared__ double sm[];
-  const int par = levStart + blockIdx.x;
-  const int ordOut = ordOf[lev], nOut = NMOM(ordOut), nIn = NMOM(ordOf[lev + 1]);
-  double *R = sm, *b = sm + nOut;
+  const int par = levStart + blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63, nk = nKids[par];
+  const int nOut = NMOM(ordOf[lev]), nIn = NMOM(ordOf[lev + 1]);
+  double *R = sm + 2 * w * nOut, *b = R + nOut;   // this wave's kid
   // the (alpha - k, k) pair table of the outputs, staged once: the inner loop
   // then reads LDS instead of waiting on global loads term by term
-  int *tS = reinterpret_cast<int *>(b + nOut), *tab = tS + nOut + 1;
+  int *tS = reinterpret_cast<int *>(sm + 16 * nOut), *tab = tS + nOut + 1;
   const int t0 = T.m2mStart[0];
-  for (int a = threadIdx.x; a <= nOut; a += blockDim.x) tS[a] = T.m2mStart[a] - t0;
-  for (int e = threadIdx.x; e < T.m2mStart[nOut] - t0; e += blockDim.x) tab[e] = T.m2m[t0 + e];
-  double acc[4] = {0, 0, 0, 0};
-  for (int k = 0; k < nKids[par]; k++) {
-    const int kid = kidStart[par] + k;
+  for (int a = threadIdx.x; a <= nOut; a += 512) tS[a] = T.m2mStart[a] - t0;
+  for (int e = threadIdx.x; e < T.m2mStart[nOut] - t0; e += 512) tab[e] = T.m2m[t0 + e];
+  if (w < nk) {
+    const int kid = kidStart[par] + w;
     double tr[3];
     for (int d = 0; d < 3; d++) tr[d] = ctx_[3 * kid + d] - ctx_[3 * par + d];
-    __syncthreads();
-    for (int a = threadIdx.x; a < nOut; a += blockDim.x) {
+    for (int a = lane; a < nOut; a += 64) {
       R[a] = conVect1(tr, T.mi[a], T.ifact3[a]);
       b[a] = a < nIn ? cmom[(long long)kid * nmMax + a] : 0.0;
     }
-    __syncthreads();
+  }
+  __syncthreads();
+  double t[4] = {0, 0, 0, 0};
+  if (w < nk)
 #pragma unroll
     for (int s = 0; s < 4; s++) {
-      const int a = threadIdx.x + s * blockDim.x;
-      if (a < nOut) {
-        double t = 0.0;
+      const int a = lane + 64 * s;
+      if (a < nOut)
         for (int e = tS[a]; e < tS[a + 1]; e++) {
           const int pr = tab[e];
-          if ((pr >> 16) < nIn) t += R[pr & 0xffff] * b[pr >> 16];
+          if ((pr >> 16) < nIn) t[s] += R[pr & 0xffff] * b[pr >> 16];
         }
-        acc[s] += t;
-      }
     }
-  }
+  __syncthreads();
+  if (w < nk)
 #pragma unroll
-  for (int s = 0; s < 4; s++) {
-    const int a = threadIdx.x + s * blockDim.x;
-    if (a < nOut) cmom[(long long)par * nmMax + a] = acc[s];
+    for (int s = 0; s < 4; s++)
+      if (lane + 64 * s < nOut) b[lane + 64 * s] = t[s];
+  __syncthreads();
+  for (int a = threadIdx.x; a < nOut; a += 512) {
+    double acc = 0.0;
+    for (int k = 0; k < nk; k++) acc += sm[2 * k * nOut + nOut + a];
+    cmom[(long long)par * nmMax + a] = acc;
   }
 }
 
@@ -4416,25 +4423,26 @@ __global__ __launch_bounds__(64) void k_adj_red_dir(int levStart, const int *__r
 }
 
 // dE/dq_j = phi_j + sum over the clusters A from j's leaf up to level height of
-// sum_a Lam_A[a] (x_j - c_A)^a / a! (the moments' monomials); one thread per
-// charge of a leaf, in the leaf's charge order
-__global__ void k_adj_eval(int levStart, const int *__restrict__ chgStart, const int *__restrict__ nChgs,
-                           const int *__restrict__ chgIdx, const int *__restrict__ parent,
-                           const int *__restrict__ level, const double *__restrict__ cx,
-                           const double *__restrict__ pos, const double *__restrict__ lam, const double *phi,
-                           int height, int P, int nmMax, DevTabs T, double *__restrict__ out) {
-  const int leaf = levStart + blockIdx.x, nm = NMOM(P);
-  for (int k = threadIdx.x; k < nChgs[leaf]; k += blockDim.x) {
+// sum_a Lam_A[a] (x_j - c_A)^a / a! (the moments' monomials); one wave per charge of
+// a leaf, lanes over a (a thread per charge left most lanes of a block idle over a
+// serial sum: 5,000 charges, 73 -> 22 us)
+__global__ __launch_bounds__(256) void k_adj_eval(int levStart, const int *__restrict__ chgStart,
+                                                  const int *__restrict__ nChgs, const int *__restrict__ chgIdx,
+                                                  const int *__restrict__ parent, const int *__restrict__ level,
+                                                  const double *__restrict__ cx, const double *__restrict__ pos,
+                                                  const double *__restrict__ lam, const double *phi, int height, int P,
+                                                  int nmMax, DevTabs T, double *__restrict__ out) {
+  const int leaf = levStart + blockIdx.x, nm = NMOM(P), w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int k = w; k < nChgs[leaf]; k += 4) {
     const int j = chgIdx[chgStart[leaf] + k];
-    double v = phi[j];
+    double s = 0.0;
     for (int A = leaf; A >= 0 && level[A] >= height; A = parent[A]) {
       const double tr[3] = {pos[3 * j] - cx[3 * A], pos[3 * j + 1] - cx[3 * A + 1], pos[3 * j + 2] - cx[3 * A + 2]};
       const double *L = lam + (long long)A * nmMax;
-      double s = 0.0;
-      for (int a = 0; a < nm; a++) s = fma(L[a], conVect1(tr, T.mi[a], T.ifact3[a]), s);
-      v += s;
+      for (int a = lane; a < nm; a += 64) s = fma(L[a], conVect1(tr, T.mi[a], T.ifact3[a]), s);
     }
-    out[j] = v;
+    s = waveSum(s);
+    if (lane == 0) out[j] = phi[j] + s;
   }
 }
 
@@ -7576,8 +7584,8 @@ static int walkCharges(fbh_ctx *c, const ChargeSet &s, int mode, double theta, c
       if (lvCount[l] <= 0) continue;
       int nOut = NMOM(ord[l]);
       const size_t lds =
-          2 * nOut * sizeof(double) + (size_t)(nOut + 1 + c->hM2mStart[nOut] - c->hM2mStart[0]) * sizeof(int);
-      hipLaunchKernelGGL(k_ct_m2m, dim3(lvCount[l]), dim3(blk64((nOut + 3) / 4, 256)), lds, strm, lvStart[l],
+          16 * nOut * sizeof(double) + (size_t)(nOut + 1 + c->hM2mStart[nOut] - c->hM2mStart[0]) * sizeof(int);
+      hipLaunchKernelGGL(k_ct_m2m, dim3(lvCount[l]), dim3(512), lds, strm, lvStart[l],
                          s.dKid, s.dNK, s.dX, s.dOrd, l, s.dMom, nmMax, c->T);
     }
     if (s.uni)   // the first enPolyW entries are the W table
@@ -7881,7 +7889,7 @@ static int adjWalk(fbh_ctx *c, const ChargeSet &s, int kind, double theta, const
 static int adjEval(fbh_ctx *c, const ChargeSet &s, const double *lamBuf, const double *phi, double *dq) {
   const int depth = c->depth;
   if (s.lvCount[depth] > 0)
-    hipLaunchKernelGGL(k_adj_eval, dim3(s.lvCount[depth]), dim3(64), 0, c->stream, s.lvStart[depth], s.dCS, s.dNC,
+    hipLaunchKernelGGL(k_adj_eval, dim3(s.lvCount[depth]), dim3(256), 0, c->stream, s.lvStart[depth], s.dCS, s.dNC,
                        s.dCI, s.dPar, s.dLevel, s.dX, s.dPos, lamBuf, phi, c->height, s.P, c->nmMax, c->T, dq);
   HCK(hipGetLastError());
   return 1;
