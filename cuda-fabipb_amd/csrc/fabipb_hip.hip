@@ -1240,31 +1240,25 @@ __global__ __launch_bounds__(64) void k_spec_vals32(const Pnl *__restrict__ pnl,
 }
 
 // LDS: (p in the destination leaf's frame, A sigma), (n, A sigma_n), source panel index; FLY_CHUNK each
-__device__ __forceinline__ void nearFly32Tile(int t, const int2 *__restrict__ tiles,
-                                              const int *__restrict__ leafStart, const int *__restrict__ leafCount,
-                                              const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
-                                              const int *__restrict__ srcList, const float4 *__restrict__ PA,
-                                              const float4 *__restrict__ PN, const float4 *__restrict__ PL,
-                                              const double *__restrict__ x, const long long *__restrict__ specOff,
-                                              const int *__restrict__ specCol, const float4 *__restrict__ specVal,
-                                              float *__restrict__ out, int n, float kappa, float eps, float4 *sP,
-                                              float4 *sN, int *sY, const int *__restrict__ ownOff) {
-  const int2 tl = tiles[t];
-  const int D = tl.x, r0 = tl.y;
-  const int oc = ownOff[D], nOwn = oc >= 0 ? leafCount[D] : 0;   // D's own columns: [oc, oc + nOwn)
-  const int rows = min(NEAR_ROWS, leafCount[D] - r0);
-  const int ncol = ncolArr[D];
-  const int *src = srcList + srcOff[D];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+__device__ __forceinline__ void nearFly32Tile(const NearTile &tl, const int *__restrict__ srcList,
+                                              const int *__restrict__ leafOf, const int *__restrict__ leafStart,
+                                              const float4 *__restrict__ PA, const float4 *__restrict__ PN,
+                                              const float4 *__restrict__ PL, const double *__restrict__ x,
+                                              const long long *__restrict__ specOff, const int *__restrict__ specCol,
+                                              const float4 *__restrict__ specVal, float *__restrict__ out, int n,
+                                              float kappa, float eps, float4 *sP, float4 *sN, int *sY) {
+  const int oc = tl.own, nOwn = tl.nOwn, rows = tl.rows, ncol = tl.ncol;   // own columns: [oc, oc + nOwn)
+  const int *src = srcList + tl.src;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const float k4pi = (float)kFourPiI, kap2 = kappa * kappa, ieps = 1.f / eps, nk = -kappa * (float)M_LOG2E;
-  const float4 O = PA[leafStart[D]];   // the leaf's frame
+  const float4 O = PA[leafStart[leafOf[tl.row0]]];   // the leaf's frame
   float4 XQ[4], XN[4];
   float XA[4];
   int xi[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int row = w + 4 * r;
-    xi[r] = leafStart[D] + r0 + min(row, rows - 1);
+    xi[r] = tl.row0 + min(row, rows - 1);
     const float4 p = PA[xi[r]];
     XA[r] = p.w;
     XQ[r] = flyLocal(p, PL[xi[r]], O);
@@ -1319,29 +1313,36 @@ __device__ __forceinline__ void nearFly32Tile(int t, const int2 *__restrict__ ti
 
 #define MIX32_LDS (2 * FLY_CHUNK * 16 + FLY_CHUNK * 4)
 static_assert(MIX32_LDS >= 2 * NEAR_CHUNK * 4, "the stream tiles' LDS must fit the union");
-__global__ __launch_bounds__(256) void k_near_mix32(const int2 *__restrict__ tiles, const int *__restrict__ leafStart,
-                                                    const int *__restrict__ leafCount,
-                                                    const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
-                                                    const long long *__restrict__ tileCoef,
-                                                    const int *__restrict__ srcList,
-                                                    const float4 *__restrict__ coef, const float4 *__restrict__ PA,
-                                                    const float4 *__restrict__ PN, const float4 *__restrict__ PL,
-                                                    const double *__restrict__ x,
-                                                    const long long *__restrict__ specOff,
-                                                    const int *__restrict__ specCol,
-                                                    const float4 *__restrict__ specVal, float *__restrict__ out, int n,
-                                                    float kappa, float eps, const int *__restrict__ order,
-                                                    const int *__restrict__ ownOff) {
+// MIX as in k_near_mix64: without it every tile is computed (the default), and the
+// kernel needs no registers for the stream.  Six waves a SIMD by the bound (its rows'
+// points and normals are wave-uniform): 317k panels, beside the far chain: 640 us at
+// 86 VGPRs (five waves), 520 so; the refined solve, which waits for the far chain as
+// well, 9.64 -> 9.54 ms (seven waves, with spills: 10.1).  Same values bit for bit.
+template <bool MIX>
+__global__ __launch_bounds__(256, 6) void k_near_mix32(const NearTile *__restrict__ desc, const int2 *__restrict__ tiles,
+                                                       const int *__restrict__ leafOf,
+                                                       const int *__restrict__ leafStart,
+                                                       const int *__restrict__ leafCount,
+                                                       const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
+                                                       const long long *__restrict__ tileCoef,
+                                                       const int *__restrict__ srcList,
+                                                       const float4 *__restrict__ coef, const float4 *__restrict__ PA,
+                                                       const float4 *__restrict__ PN, const float4 *__restrict__ PL,
+                                                       const double *__restrict__ x,
+                                                       const long long *__restrict__ specOff,
+                                                       const int *__restrict__ specCol,
+                                                       const float4 *__restrict__ specVal, float *__restrict__ out,
+                                                       int n, float kappa, float eps) {
   __shared__ __align__(16) unsigned char lds[MIX32_LDS];
-  const int t = order[blockIdx.x];   // costliest tiles first
-  if (tileCoef[t] >= 0) {
+  const NearTile tl = desc[blockIdx.x];   // costliest tiles first
+  if (MIX && tileCoef[tl.tile] >= 0) {
     float *sS = reinterpret_cast<float *>(lds);
-    nearStreamTile<float>(t, tiles, leafStart, leafCount, srcOff, ncolArr, tileCoef, srcList, coef, x, out, n, sS,
+    nearStreamTile<float>(tl.tile, tiles, leafStart, leafCount, srcOff, ncolArr, tileCoef, srcList, coef, x, out, n, sS,
                           sS + NEAR_CHUNK);
   } else {
     float4 *sP = reinterpret_cast<float4 *>(lds);
-    nearFly32Tile(t, tiles, leafStart, leafCount, srcOff, ncolArr, srcList, PA, PN, PL, x, specOff, specCol, specVal,
-                  out, n, kappa, eps, sP, sP + FLY_CHUNK, reinterpret_cast<int *>(sP + 2 * FLY_CHUNK), ownOff);
+    nearFly32Tile(tl, srcList, leafOf, leafStart, PA, PN, PL, x, specOff, specCol, specVal, out, n, kappa, eps, sP,
+                  sP + FLY_CHUNK, reinterpret_cast<int *>(sP + 2 * FLY_CHUNK));
   }
 }
 
@@ -4718,10 +4719,7 @@ struct fbh_ctx {
   size_t m2lLds = 0;
   int m2lWaves = 0;
   int m2lMaxT = 0;   // register-resident term lists (16, 32) or 0
-  // FP64 mixed nearfield launch: tiles costliest first, grid-stride over them
-  int *tileOrder = nullptr;
-  int nearGrid = 0;
-  int *ownOff = nullptr;   // per leaf: the column of its own first panel in its column list (-1: none)
+  int nearGrid = 0;   // blocks of the FP64 nearfield launch (fewer than the tiles: grid-stride over them)
   // M2L term grid (k_m2l_grid): K steps x 64 lanes per order, runs of L steps
   int gridK = 0, gridL = 0, gridSlotZ = 0, gridNcc = 0, gridNgg = 0, gridWaves = 4;
   unsigned *gridTerms = nullptr;
@@ -5665,9 +5663,7 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
       desc[k] = {leafStart[D] + r0, std::min(NEAR_ROWS, leafCount[D] - r0), srcOff[D], ncol[D], std::max(ownOff[D], 0),
                  ownOff[D] >= 0 ? leafCount[D] : 0, t, 0};
     }
-    if (!(c->tileOrder = dupload(c, order.data(), order.size())) || !(c->ownOff = dupload(c, ownOff.data(), ownOff.size())) ||
-        !(c->nearDesc = dupload(c, desc.data(), desc.size())))
-      FAIL();
+    if (!(c->nearDesc = dupload(c, desc.data(), desc.size()))) FAIL();
     // blocks of the FP64 nearfield launch (0: one per tile, the fastest here;
     // resident grids of 2-4 blocks per CU were slower beside the far chain)
     const char *eg = getenv("FABIPB_NEAR_GRID");
@@ -6063,11 +6059,16 @@ static void nearPass(fbh_ctx *c, const OpBufs<R> &B, const double *x, hipStream_
   if (c->nFlyTiles > 0) {
     if constexpr (std::is_same<R, double>::value)
       nearMix64(c, B.coef, c->specVal64, x, 0, st);
-    else
-      hipLaunchKernelGGL(k_near_mix32, dim3(c->nTiles), dim3(256), c->near32Pad, st, c->tiles, c->leafStart, c->leafCount,
-                         c->srcOff, c->ncol, c->tileCoef, c->srcList, B.coef, c->flyPA, c->flyPN, c->flyPL, x,
-                         c->specOff, c->specCol, c->specVal, B.nearv, c->n, (float)c->kappa, (float)c->eps, c->tileOrder,
-                         c->ownOff);
+    else {
+      auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(c->nTiles), dim3(256), c->near32Pad, st, c->nearDesc, c->tiles, c->leafOf,
+                           c->leafStart, c->leafCount, c->srcOff, c->ncol, c->tileCoef, c->srcList, B.coef, c->flyPA,
+                           c->flyPN, c->flyPL, x, c->specOff, c->specCol, c->specVal, B.nearv, c->n, (float)c->kappa,
+                           (float)c->eps);
+      };
+      if (c->nStored > 0) launch(k_near_mix32<true>);
+      else launch(k_near_mix32<false>);
+    }
     return;
   }
   hipLaunchKernelGGL(k_near_apply<R>, dim3(c->nTiles), dim3(256), 0, st, c->tiles, c->leafStart, c->leafCount,
