@@ -6777,7 +6777,8 @@ static int ensureGmres(fbh_ctx *c, int restart) {
     if (c->hpin) hipHostFree(c->hpin);
     c->hpin = nullptr;
     c->hpinLen = 0;
-    HCK(hipHostMalloc((void **)&c->hpin, (restart + 8) * sizeof(double), hipHostMallocDefault));
+    // coherent: kernels store into it and the host reads after an event, whose release need not reach the system
+    HCK(hipHostMalloc((void **)&c->hpin, (restart + 8) * sizeof(double), hipHostMallocCoherent));
     c->hpinLen = restart + 8;
   }
   if (!c->evDone) HCK(hipEventCreateWithFlags(&c->evDone, hipEventDisableTiming));
