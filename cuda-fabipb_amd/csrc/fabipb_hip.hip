@@ -611,13 +611,12 @@ template <> struct Vec4<float> { typedef float4 type; };
 // sources of K0*sgm_n + K1*sgm, out[x+n] = K2*sgm_n + K3*sgm.  R is the
 // arithmetic of the coefficients, the staged densities and the sums.  The
 // tile's coefficient rows start at tileCoef[t] (row stride = the leaf's
-// column count).  HBM bounds it.  TOGETHER: a wave
-// streams its four rows together (rows past the tile repeat its last one), eight loads
-// a lane in flight where a row at a time keeps two; 20,480 panels at q = 2 (26M pairs,
-// 844 MB): 169 -> 161 us beside the far chain, matvec 183.4 -> 178.4.  Not in the
-// kernels that hold computed tiles too, which its registers cost a resident block
-// (k_near_mix32, 317k panels: 627 -> 690 us).
-template <typename R, bool TOGETHER = false>
+// column count).  HBM bounds it.  A wave takes its rows one after another: its four
+// together (eight loads a lane in flight, 151 VGPRs in FP64 against 83) gain only where
+// leaves are large (20,480 panels, q = 2, depth 2: matvec 712 us a row at a time, 681
+// together; depth 3: 210, 208) and lose elsewhere (depth 4: 126, 127; depth 5: 235, 240;
+// 81,920 panels, depth 4: 631, 639; the dense operator of 5,120 panels: 153, 173).
+template <typename R>
 __device__ __forceinline__ void nearStreamTile(int t, const int2 *__restrict__ tiles,
                                                const int *__restrict__ leafStart, const int *__restrict__ leafCount,
                                                const int *__restrict__ srcOff, const int *__restrict__ ncolArr,
@@ -644,69 +643,29 @@ __device__ __forceinline__ void nearStreamTile(int t, const int2 *__restrict__ t
       sN[j] = (R)x[y + n];
     }
     __syncthreads();
-    if constexpr (TOGETHER) {
-      if (w < rows) {
-        const R4 *cr[4];
-        R s0[4] = {0, 0, 0, 0}, s1[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int r = 0; r < 4; r++) cr[r] = cbase + (long long)min(w + 4 * r, rows - 1) * ncol + c0;
+    for (int r = 0; r < 4; r++) {
+      const int row = w + 4 * r;
+      if (row < rows) {
+        const R4 *cr = cbase + (long long)row * ncol + c0;
+        R s0 = 0, s1 = 0;
         int j = lane;
         for (; j + 64 < cn; j += 128) {
-          R4 c[4], d[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            c[r] = cr[r][j];
-            d[r] = cr[r][j + 64];
-          }
-          const R p = sS[j], m = sN[j], p2 = sS[j + 64], m2 = sN[j + 64];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            s0[r] += c[r].x * m + c[r].y * p;
-            s1[r] += c[r].z * m + c[r].w * p;
-            s0[r] += d[r].x * m2 + d[r].y * p2;
-            s1[r] += d[r].z * m2 + d[r].w * p2;
-          }
+          R4 c = cr[j], d = cr[j + 64];
+          R p = sS[j], m = sN[j], p2 = sS[j + 64], m2 = sN[j + 64];
+          s0 += c.x * m + c.y * p;
+          s1 += c.z * m + c.w * p;
+          s0 += d.x * m2 + d.y * p2;
+          s1 += d.z * m2 + d.w * p2;
         }
         if (j < cn) {
-          const R p = sS[j], m = sN[j];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const R4 c = cr[r][j];
-            s0[r] += c.x * m + c.y * p;
-            s1[r] += c.z * m + c.w * p;
-          }
+          R4 c = cr[j];
+          R p = sS[j], m = sN[j];
+          s0 += c.x * m + c.y * p;
+          s1 += c.z * m + c.w * p;
         }
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          a0[r] += s0[r];
-          a1[r] += s1[r];
-        }
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = w + 4 * r;
-        if (row < rows) {
-          const R4 *cr = cbase + (long long)row * ncol + c0;
-          R s0 = 0, s1 = 0;
-          int j = lane;
-          for (; j + 64 < cn; j += 128) {
-            R4 c = cr[j], d = cr[j + 64];
-            R p = sS[j], m = sN[j], p2 = sS[j + 64], m2 = sN[j + 64];
-            s0 += c.x * m + c.y * p;
-            s1 += c.z * m + c.w * p;
-            s0 += d.x * m2 + d.y * p2;
-            s1 += d.z * m2 + d.w * p2;
-          }
-          if (j < cn) {
-            R4 c = cr[j];
-            R p = sS[j], m = sN[j];
-            s0 += c.x * m + c.y * p;
-            s1 += c.z * m + c.w * p;
-          }
-          a0[r] += s0;
-          a1[r] += s1;
-        }
+        a0[r] += s0;
+        a1[r] += s1;
       }
     }
   }
@@ -731,7 +690,7 @@ __global__ __launch_bounds__(256) void k_near_apply(const int2 *__restrict__ til
                                                     const typename Vec4<R>::type *__restrict__ coef,
                                                     const double *__restrict__ x, R *__restrict__ out, int n) {
   __shared__ R sS[NEAR_CHUNK], sN[NEAR_CHUNK];
-  nearStreamTile<R, true>(blockIdx.x, tiles, leafStart, leafCount, srcOff, ncolArr, tileCoef, srcList, coef, x, out, n,
+  nearStreamTile<R>(blockIdx.x, tiles, leafStart, leafCount, srcOff, ncolArr, tileCoef, srcList, coef, x, out, n,
                     sS, sN);
 }
 
