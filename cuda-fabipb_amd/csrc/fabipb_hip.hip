@@ -1208,7 +1208,7 @@ __device__ __forceinline__ void nearFly32Tile(const NearTile &tl, const int *__r
                                               float kappa, float eps, float4 *sP, float4 *sN, int *sY) {
   const int oc = tl.own, nOwn = tl.nOwn, rows = tl.rows, ncol = tl.ncol;   // own columns: [oc, oc + nOwn)
   const int *src = srcList + tl.src;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float k4pi = (float)kFourPiI, kap2 = kappa * kappa, ieps = 1.f / eps, nk = -kappa * (float)M_LOG2E;
   const float4 O = PA[leafStart[leafOf[tl.row0]]];   // the leaf's frame
   float4 XQ[4], XN[4];
@@ -1273,12 +1273,18 @@ __device__ __forceinline__ void nearFly32Tile(const NearTile &tl, const int *__r
 #define MIX32_LDS (2 * FLY_CHUNK * 16 + FLY_CHUNK * 4)
 static_assert(MIX32_LDS >= 2 * NEAR_CHUNK * 4, "the stream tiles' LDS must fit the union");
 // MIX as in k_near_mix64: without it every tile is computed (the default), and the
-// kernel needs no registers for the stream.  Six waves a SIMD by the bound (its rows'
-// points and normals are wave-uniform): 317k panels, beside the far chain: 640 us at
-// 86 VGPRs (five waves), 520 so; the refined solve, which waits for the far chain as
-// well, 9.64 -> 9.54 ms (seven waves, with spills: 10.1).  Same values bit for bit.
+// kernel needs no registers for the stream.  The rows' points and normals stay in the
+// lanes' registers: read as scalars (the wave's number made uniform) they leave 56 VGPRs
+// and room for eight waves a SIMD, but an FP32 instruction takes one scalar operand and
+// the copies cost more than the waves bring (20,480 panels, depth 2, alone: 127 us so,
+// 145 with scalars), and blocks that hold every wave slot starve the far chain beside
+// them (its M2M needs eight slots of a CU at once).  Five waves a SIMD by the bound,
+// 84 VGPRs; product in FP32, so against scalars: 81,920 panels, order 4: 160 us, 173;
+// order 6: 184, 192; depth 5: 232, 246; 20,480, depth 2: 151, 169; 317k panels: order 4:
+// 556, 570; only order 6 is the other way, 644, 635.  Six waves (80 VGPRs) win a little
+// at 317k (635) and lose at depth 2 (157) and depth 5 (239).  Same values bit for bit.
 template <bool MIX>
-__global__ __launch_bounds__(256, 6) void k_near_mix32(const NearTile *__restrict__ desc, const int2 *__restrict__ tiles,
+__global__ __launch_bounds__(256, 5) void k_near_mix32(const NearTile *__restrict__ desc, const int2 *__restrict__ tiles,
                                                        const int *__restrict__ leafOf,
                                                        const int *__restrict__ leafStart,
                                                        const int *__restrict__ leafCount,
