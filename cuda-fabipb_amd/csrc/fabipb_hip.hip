@@ -3834,13 +3834,15 @@ __device__ __forceinline__ void enFar32(const float *__restrict__ co0, double rx
 #define EN_TARGET_WAVES 8192   // slices are added until the walk has this many waves
 #endif
 // waves per SIMD the walk's registers must allow: 4 (a few spilled registers in
-// the energy's modes), 3 for those at orders 8 and 9 (53 and 67 spills at four),
-// the compiler's choice for MODE 4
-__host__ __device__ constexpr int enMinWaves(int mode, int p) {
-  return mode == 4 ? 1 : mode != 1 && p >= 8 ? 3 : 4;
+// the energy's modes), 3 for the FP64 ones at orders 8 and 9 (53 and 67 spills at four),
+// the compiler's choice for MODE 4.  The FP32 form spills 0 and 4 registers at four waves
+// and orders 8 and 9: 81,920 panels, 5,000 charges, 1,122 us with three waves against
+// 1,031 at order 8, 1,610 against 1,435 at order 9.
+__host__ __device__ constexpr int enMinWaves(int mode, int p, bool f32) {
+  return f32 ? 4 : mode == 4 ? 1 : mode != 1 && p >= 8 ? 3 : 4;
 }
 template <int P, int MODE, typename R = double>
-__global__ __launch_bounds__(64 * EN_WPB, enMinWaves(MODE, P)) void k_energy_wave(const Pnl *__restrict__ pnl, int n, const double *__restrict__ sgm,
+__global__ __launch_bounds__(64 * EN_WPB, enMinWaves(MODE, P, sizeof(R) == 4)) void k_energy_wave(const Pnl *__restrict__ pnl, int n, const double *__restrict__ sgm,
                                                      const int *__restrict__ level, const double *__restrict__ cx,
                                                      const double *__restrict__ eRad,
                                                      const int *__restrict__ kidStart, const int *__restrict__ nKids,
