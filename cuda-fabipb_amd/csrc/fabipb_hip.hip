@@ -3835,11 +3835,15 @@ __device__ __forceinline__ void enFar32(const float *__restrict__ co0, double rx
 #endif
 // waves per SIMD the walk's registers must allow: 4 (a few spilled registers in
 // the energy's modes), 3 for the FP64 ones at orders 8 and 9 (53 and 67 spills at four),
-// the compiler's choice for MODE 4.  The FP32 form spills 0 and 4 registers at four waves
-// and orders 8 and 9: 81,920 panels, 5,000 charges, 1,122 us with three waves against
+// the compiler's choice for MODE 4 up to order 7 (two waves from order 3 on; three spill
+// and measure the same), 2 above (33 and 55 spills): left to the compiler it took 291 and
+// 314 registers, one wave a SIMD; a gradient with one adjoint step, one wave against two:
+// 81,920 panels, 5,000 charges, order 8: 5,775 us, 5,390; order 9: 10,830, 10,340; the
+// 163,840-panel shell, 30,000 charges, order 8: 21.0 ms, 18.5 (three waves: 19.0).
+// The FP32 form spills 0 and 4 registers at four waves and orders 8 and 9: 81,920 panels, 5,000 charges, 1,122 us with three waves against
 // 1,031 at order 8, 1,610 against 1,435 at order 9.
 __host__ __device__ constexpr int enMinWaves(int mode, int p, bool f32) {
-  return f32 ? 4 : mode == 4 ? 1 : mode != 1 && p >= 8 ? 3 : 4;
+  return f32 ? 4 : mode == 4 ? (p >= 8 ? 2 : 1) : mode != 1 && p >= 8 ? 3 : 4;
 }
 template <int P, int MODE, typename R = double>
 __global__ __launch_bounds__(64 * EN_WPB, enMinWaves(MODE, P, sizeof(R) == 4)) void k_energy_wave(const Pnl *__restrict__ pnl, int n, const double *__restrict__ sgm,

@@ -39,6 +39,7 @@ def waves(built, tmp_path_factory):
     ("k_near_apply", "IdE", 5), ("k_near_apply", "IfE", 8),
     ("k_near_mix32", "ILb0E", 5),
     ("k_energy_wave", "ILi8ELi0EfE", 4), ("k_energy_wave", "ILi9ELi0EfE", 4),
+    ("k_energy_wave", "ILi8ELi4EdE", 2), ("k_energy_wave", "ILi9ELi4EdE", 2),
 ])
 def test_waves_per_simd(waves, name, args, want):
     assert waves(name, args) == want
