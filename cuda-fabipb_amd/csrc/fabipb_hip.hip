@@ -4763,7 +4763,6 @@ struct fbh_ctx {
   int gmRestart = 0;
   double *V = nullptr, *w = nullptr, *r = nullptr, *part = nullptr, *hcol = nullptr, *ydev = nullptr, *scal = nullptr;
   double *hpin = nullptr;   // pinned host staging of the small readbacks (norms, Hessenberg columns, y)
-  int hpinLen = 0;
   hipEvent_t evDone = nullptr;   // marks a readback; the host spins on it
 };
 
@@ -6733,25 +6732,27 @@ extern "C" int fbh_psolve_dev(fbh_ctx *c, double *out, const double *in) {
 
 static int ensureGmres(fbh_ctx *c, int restart) {
   if (c->V && c->gmRestart >= restart) return 1;
-  if (c->V) { hipFree(c->V); c->V = nullptr; }
+  // kernels store into these buffers by address, so a growth that fails part-way must
+  // leave no freed pointer behind and must not pass as ready for a shorter restart
+  c->gmRestart = 0;
+  auto drop = [](double *&p, bool pinned) {
+    if (p) pinned ? hipHostFree(p) : hipFree(p);
+    p = nullptr;
+  };
+  drop(c->V, false);
+  drop(c->hcol, false);
+  drop(c->ydev, false);
+  drop(c->hpin, true);
   size_t n2 = 2 * (size_t)c->n;
   HCK(hipMalloc(&c->V, n2 * (restart + 1) * sizeof(double)));
   if (!c->w) HCK(hipMalloc(&c->w, n2 * sizeof(double)));
   if (!c->r) HCK(hipMalloc(&c->r, n2 * sizeof(double)));
   if (!c->part) HCK(hipMalloc(&c->part, 2 * RED_BLOCKS * sizeof(double)));   // two sets (ping-pong)
-  if (c->hcol) hipFree(c->hcol);
-  if (c->ydev) hipFree(c->ydev);
   HCK(hipMalloc(&c->hcol, (restart + 2) * sizeof(double)));
   HCK(hipMalloc(&c->ydev, (restart + 2) * sizeof(double)));
   if (!c->scal) HCK(hipMalloc(&c->scal, 4 * sizeof(double)));
-  if (c->hpinLen < restart + 8) {
-    if (c->hpin) hipHostFree(c->hpin);
-    c->hpin = nullptr;
-    c->hpinLen = 0;
-    // coherent: kernels store into it and the host reads after an event, whose release need not reach the system
-    HCK(hipHostMalloc((void **)&c->hpin, (restart + 8) * sizeof(double), hipHostMallocCoherent));
-    c->hpinLen = restart + 8;
-  }
+  // coherent: kernels store into it and the host reads after an event, whose release need not reach the system
+  HCK(hipHostMalloc((void **)&c->hpin, (restart + 8) * sizeof(double), hipHostMallocCoherent));
   if (!c->evDone) HCK(hipEventCreateWithFlags(&c->evDone, hipEventDisableTiming));
   c->gmRestart = restart;
   return 1;
