@@ -4695,6 +4695,7 @@ struct fbh_ctx {
   int gridK = 0, gridL = 0, gridSlotZ = 0, gridNcc = 0, gridNgg = 0, gridWaves = 4;
   unsigned *gridTerms = nullptr;
   int *m2lOrder = nullptr;     // cubes by interaction-list length, longest first
+  std::vector<int> hM2lOrder;  // (host copy)
   int gmShape = -1, gmGroups = 1;   // the FP64 M2L by tensor slot (k_m2l_gamma): shape, groups per block
   GammaPlans gmPlans = {};
   GammaCube *gmCubes = nullptr;
@@ -4788,6 +4789,33 @@ static T *dupload(fbh_ctx *c, const T *h, size_t count) {
     return nullptr;
   }
   return d;
+}
+
+// several host arrays in one allocation and one copy, each on a 256-byte boundary: a
+// small copy costs about 15 us by itself
+struct Upload {
+  void *dev;   // the address of the device pointer
+  const void *host;
+  size_t bytes;
+  template <class T>
+  Upload(T **d, const T *h, size_t count) : dev(d), host(h), bytes(count * sizeof(T)) {}
+};
+static bool uploadAll(fbh_ctx *c, std::initializer_list<Upload> ups) {
+  size_t total = 0;
+  for (const Upload &u : ups) total += (u.bytes + 255) & ~(size_t)255;
+  std::vector<unsigned char> stage(total);
+  unsigned char *h = stage.data();
+  for (const Upload &u : ups) {
+    if (u.bytes) memcpy(h, u.host, u.bytes);
+    h += (u.bytes + 255) & ~(size_t)255;
+  }
+  unsigned char *d = dupload(c, stage.data(), total);
+  if (!d) return false;
+  for (const Upload &u : ups) {
+    memcpy(u.dev, &d, sizeof d);
+    d += (u.bytes + 255) & ~(size_t)255;
+  }
+  return true;
 }
 
 // The panel pass of the FMM tree on the device (src/gkSetup.c:90-301): each
@@ -5246,7 +5274,8 @@ static bool planGrid(const fbh_ctx *c, int p, int K, int L, int slotZ, std::vect
 // The term grid for every order the levels use, on the smallest compiled shape
 // (K, L) that holds the largest of them; none above order 8 (k_m2l_cached then).
 static bool buildM2LGrid(fbh_ctx *c) {
-  std::vector<int> order(c->nCube);   // cubes by interaction-list length, longest first
+  std::vector<int> &order = c->hM2lOrder;   // cubes by interaction-list length, longest first
+  order.resize(c->nCube);
   for (int i = 0; i < c->nCube; i++) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
     return c->hM2lOff[a + 1] - c->hM2lOff[a] > c->hM2lOff[b + 1] - c->hM2lOff[b];
@@ -5328,13 +5357,21 @@ static bool planGamma(int p, int L, int W, int slotZ, HostGamma &H) {
         mi[3 * g + 1] = i2;
         mi[3 * g + 2] = d - i1 - i2;
       }
-  std::vector<std::vector<int>> pool(nm);
-  std::vector<int> size;
+  // pool: every gamma's betas not yet placed, in graded order, at [poolOff[g], + poolLen[g])
+  std::vector<int> pool, poolOff(nm), poolLen(nm), size;
+  pool.reserve((size_t)L * cells);
+  size.reserve(cells);
   H.gamma.clear();
+  H.gamma.reserve(cells);
   for (int g = 0; g < nm; g++) {
-    for (int b = 0; b < nm; b++)
-      if (mi[3 * b] <= mi[3 * g] && mi[3 * b + 1] <= mi[3 * g + 1] && mi[3 * b + 2] <= mi[3 * g + 2]) pool[g].push_back(b);
-    const int m = (int)pool[g].size(), k = (m + L - 1) / L;
+    poolOff[g] = (int)pool.size();
+    const int *G = &mi[3 * g], deg = G[0] + G[1] + G[2];
+    for (int d = 0; d <= deg; d++)
+      for (int i1 = std::max(0, d - G[1] - G[2]); i1 <= std::min(d, G[0]); i1++) {
+        const int row = idx3of(i1, 0, d - i1);
+        for (int i2 = std::max(0, d - i1 - G[2]); i2 <= std::min(d - i1, G[1]); i2++) pool.push_back(row + i2);
+      }
+    const int m = poolLen[g] = (int)pool.size() - poolOff[g], k = (m + L - 1) / L;
     for (int i = 0; i < k; i++) {   // even shares
       H.gamma.push_back(g);
       size.push_back(m / k + (i < m % k));
@@ -5345,7 +5382,10 @@ static bool planGamma(int p, int L, int W, int slotZ, HostGamma &H) {
   H.gamma.resize(cells, 0);
   size.resize(cells, 0);
   H.beta.assign((size_t)L * cells, (unsigned short)slotZ);
-  std::vector<std::vector<int>> byAlpha(nm);
+  std::vector<int> count(nm), alphaOf;   // an alpha's products; the alpha of each entry (step, cell)
+  std::vector<unsigned short> entry;
+  alphaOf.reserve(pool.size());
+  entry.reserve(pool.size());
   // of the group's lanes placed in this step: how many read each bank, and how many each slot
   std::vector<int> bank(16), same(nm);
   for (int l = 0; l < L; l++) {
@@ -5355,27 +5395,30 @@ static bool planGamma(int p, int L, int W, int slotZ, HostGamma &H) {
         std::fill(same.begin(), same.end(), 0);
       }
       if (size[i] <= l) continue;
-      auto &pl = pool[H.gamma[i]];
-      size_t best = 0;
-      int bc = 1 << 30;
-      for (size_t q = 0; q < pl.size() && bc > 0; q++) {
+      const int g = H.gamma[i];
+      int *pl = &pool[poolOff[g]], best = 0, bc = 1 << 30;
+      for (int q = 0; q < poolLen[g] && bc > 0; q++) {
         const int n = bank[pl[q] % 16] - same[pl[q]];
         if (n < bc) { bc = n; best = q; }
       }
-      const int b = pl[best], g = H.gamma[i];
+      const int b = pl[best];
       bank[b % 16]++;
       same[b]++;
-      pl.erase(pl.begin() + best);
+      std::copy(pl + best + 1, pl + poolLen[g], pl + best);
+      poolLen[g]--;
       H.beta[(size_t)l * cells + i] = (unsigned short)b;
-      byAlpha[idx3of(mi[3 * g] - mi[3 * b], mi[3 * g + 1] - mi[3 * b + 1], mi[3 * g + 2] - mi[3 * b + 2])].push_back(l * cells + i);
+      alphaOf.push_back(idx3of(mi[3 * g] - mi[3 * b], mi[3 * g + 1] - mi[3 * b + 1], mi[3 * g + 2] - mi[3 * b + 2]));
+      entry.push_back((unsigned short)(l * cells + i));
+      count[alphaOf.back()]++;
     }
   }
   H.alphaSeg.assign(1, 0);
-  H.ent.clear();
-  for (int a = 0; a < nm; a++) {
-    for (int e : byAlpha[a]) H.ent.push_back((unsigned short)e);
-    while (H.ent.size() % GAMMA_SEG) H.ent.push_back((unsigned short)(L * cells));
-    H.alphaSeg.push_back((int)H.ent.size() / GAMMA_SEG);
+  for (int a = 0; a < nm; a++) H.alphaSeg.push_back(H.alphaSeg[a] + (count[a] + GAMMA_SEG - 1) / GAMMA_SEG);
+  H.ent.assign((size_t)GAMMA_SEG * H.alphaSeg[nm], (unsigned short)(L * cells));
+  std::fill(count.begin(), count.end(), 0);
+  for (size_t e = 0; e < entry.size(); e++) {
+    const int a = alphaOf[e];
+    H.ent[(size_t)GAMMA_SEG * H.alphaSeg[a] + count[a]++] = entry[e];
   }
   return true;
 }
@@ -5422,12 +5465,10 @@ static bool buildGamma(fbh_ctx *c) {
   const int gr = W == 1 ? 4 : W == 4 && c->nCube < 1024 ? 2 : 1;
   const size_t lds = std::max((size_t)gr * 4 * NB * (nmU + 1) * sizeof(double2), redLen * sizeof(double));
   if (lds > (size_t)c->ldsMax || maxSeg > 64 * W * gr) return true;
-  std::vector<GammaCube> cubes(c->nCube);   // longest interaction lists first
-  for (int i = 0; i < c->nCube; i++) cubes[i].cube = i;
-  std::stable_sort(cubes.begin(), cubes.end(), [&](const GammaCube &a, const GammaCube &b) {
-    return c->hM2lOff[a.cube + 1] - c->hM2lOff[a.cube] > c->hM2lOff[b.cube + 1] - c->hM2lOff[b.cube];
-  });
-  for (GammaCube &q : cubes) {
+  std::vector<GammaCube> cubes(c->nCube);
+  for (int i = 0; i < c->nCube; i++) {
+    GammaCube &q = cubes[i];
+    q.cube = c->hM2lOrder[i];
     q.b0 = c->hM2lOff[q.cube];
     q.b1 = c->hM2lOff[q.cube + 1];
     q.p = c->ordM2L[c->cubeLevel[q.cube]];
@@ -5553,12 +5594,13 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
   for (int l = 0; l < nLeaf; l++)
     for (int j = 0; j < leafCount[l]; j++) leafOf[leafStart[l] + j] = l;
   if (!(c->pnl = dupload(c, hp.data(), n)) || !(c->area = dupload(c, area, n)) ||
-      !(c->leafOf = dupload(c, leafOf.data(), n)) || !(c->leafStart = dupload(c, leafStart, nLeaf)) ||
-      !(c->leafCount = dupload(c, leafCount, nLeaf)) || !(c->cubeX = dupload(c, cubeX, 3 * (size_t)nCube)) ||
-      !(c->cubeLevelD = dupload(c, cubeLevel, nCube)) || !(c->kidStart = dupload(c, kidStart, nCube)) ||
-      !(c->nKids = dupload(c, nKids, nCube)) || !(c->parent = dupload(c, parent, nCube)) ||
-      !(c->m2lOff = dupload(c, m2lOff, nCube + 1)) || !(c->m2lSrc = dupload(c, m2lSrc, std::max(1, m2lOff[nCube]))) ||
-      !(c->ordMomD = dupload(c, ordMom, depth + 1)) || !(c->ordM2LD = dupload(c, ordM2L, depth + 1)))
+      !(c->leafOf = dupload(c, leafOf.data(), n)) ||
+      !uploadAll(c, {{&c->leafStart, leafStart, (size_t)nLeaf}, {&c->leafCount, leafCount, (size_t)nLeaf},
+                     {&c->cubeX, cubeX, 3 * (size_t)nCube}, {&c->cubeLevelD, cubeLevel, (size_t)nCube},
+                     {&c->kidStart, kidStart, (size_t)nCube}, {&c->nKids, nKids, (size_t)nCube},
+                     {&c->parent, parent, (size_t)nCube}, {&c->m2lOff, m2lOff, (size_t)nCube + 1},
+                     {&c->m2lSrc, m2lSrc, (size_t)std::max(1, m2lOff[nCube])},
+                     {&c->ordMomD, ordMom, (size_t)depth + 1}, {&c->ordM2LD, ordM2L, (size_t)depth + 1}}))
     FAIL();
   c->nM2L = m2lOff[nCube];
   c->nLinks = 0;
@@ -5699,10 +5741,9 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
       seen += inter;
     }
   }
-  if (!(c->srcOff = dupload(c, srcOff.data(), nLeaf + 1)) || !(c->ncol = dupload(c, ncol.data(), nLeaf)) ||
-      !(c->srcList = dupload(c, srcList.data(), srcList.size())) ||
-      !(c->tiles = dupload(c, tiles.data(), tiles.size())) ||
-      !(c->tileCoef = dupload(c, tileCoef.data(), tiles.size())) ||
+  if (!uploadAll(c, {{&c->srcOff, srcOff.data(), (size_t)nLeaf + 1}, {&c->ncol, ncol.data(), (size_t)nLeaf},
+                     {&c->srcList, srcList.data(), srcList.size()}, {&c->tiles, tiles.data(), tiles.size()},
+                     {&c->tileCoef, tileCoef.data(), tiles.size()}}) ||
       !(c->coef = dalloc<double4>(c, (size_t)std::max<long long>(c->nStored, 1))))
     FAIL();
   if (c->nStored > 0) {
