@@ -9,29 +9,34 @@
 //                   (Q2M0 moments, Q2M1 noments; L2P uses the same, fmm.c:457)
 //   mom[nCube][2][nm], lec[nCube][4][nm]   multipole / local expansions
 //   coef            nearfield Galerkin coefficients KER[4] per (dst, src)
-//                   panel pair, row-major per destination leaf: for leaf D the
-//                   rows are its panels, the columns the concatenated panels
-//                   of D's near leaves (srcList), so a row is one contiguous
-//                   stream of 32-byte records
+//                   panel pair of the tiles that stream them, row-major per
+//                   16-row tile of a destination leaf D: the columns are the
+//                   concatenated panels of D's near leaves (srcList), so a row
+//                   is one contiguous stream of 32-byte records
 //
-// Kernels (FP64 throughout):
+// Kernels (FP64; those the FP32 operator runs instead in brackets):
 //   k_q2m_mats   setup: leaf moment/noment columns, one wave per panel
 //   k_near_build setup: KER4 Galerkin quadrature per pair (disjoint Duffy rule
-//                and the Sauter-Schwab vertex/edge/self rules), one block per
-//                destination panel
-//   k_near_apply one block per 16-row tile of a destination leaf; the
-//                sources' densities are staged in LDS once per tile, each wave
-//                streams four rows of coefficients (HBM-bound)
-//   k_q2m        four waves split a leaf's panels, lanes over multi-indices
-//   k_m2m, k_l2l thread per multi-index, translation tables in LDS
-//   k_m2l_cached per destination cube, (alpha, beta) terms balanced over the
-//                lanes by a host plan, derivative tensors cached per pair
-//                (k_m2l recomputes them when the cache does not fit)
-//   k_l2p        eight lanes per panel
-//   the nearfield runs on a second stream beside the far-field chain
-//   k_combine    y = alpha*(D x - far - near) + beta*y
-//   k_rhs        direct right-hand side, thread per panel, charges in LDS
-//   k_energy     panel-tree energy, one wave per panel walking the charge tree
+//                and the Sauter-Schwab vertex/edge/self rules)
+//   k_near_mix64 [k_near_mix32] the nearfield at q = 1: one block per 16-row
+//                tile, every pair on the fly, self and shared-vertex pairs by
+//                stored corrections
+//   k_near_apply the nearfield where every tile streams its coefficients
+//   k_q2m64 [k_q2m] a block per leaf, its waves over the panels, lanes over
+//                multi-indices
+//   k_m2m_ax     a block per parent, a wave per child, one axis at a time
+//                (k_m2m, k_l2l: level by level for the stage calls)
+//   k_m2l_gamma [k_m2l_grid] per destination cube, derivative tensors cached
+//                per pair (k_m2l_cached at order 9, k_m2l where the cache does
+//                not fit)
+//   k_l2lp64 [k_l2lp] a block per leaf: L2L down its ancestry, then L2P (k_l2p
+//                alone after the stage calls' L2L)
+//   the nearfield runs on a second stream beside the far-field chain, small FP64
+//   products on one stream
+//   k_combine    y = alpha*(D x - far - near) + beta*y (one stream: in k_l2lp64)
+//   k_rhs_q1, k_rhs direct right-hand side, lanes over panels
+//   k_energy_wave right-hand side, energy and their derivatives by the charge
+//                tree, one lane per panel (k_energy: mixed orders)
 //   GMRES helpers: fixed-grid deterministic dot products, MGS update,
 //                normalisation, diagonal preconditioner, x += V y
 #include <hip/hip_runtime.h>
@@ -833,10 +838,10 @@ __device__ __forceinline__ void fly64Cols(int j0, int j1, int lane, int w, int r
 // second, 72 % of its nominal clock's rate), so the split aims at the fewest
 // instructions per pair: wave w owns rows w, w + 4, w + 8, w + 12 and takes each
 // staged source (56 bytes of LDS) once for all four, their nine sums in
-// registers.  317k panels, alone: 988 us with kernelKER4's operation order, two
-// rows per pass and the corrections added row by row at the end; 1,078 us with
-// these sums but the corrections still there; 788 us so (81,920 panels: 262 ->
-// 212 us).  On a bare copy of the loop (3.9e8 pairs): four rows 769 us, two 809,
+// registers.  317k panels, alone and back to back: 988 us with kernelKER4's operation
+// order, two rows per pass and the corrections added row by row at the end; 1,078 us with
+// these sums but the corrections still there; 788 us so (81,920 panels: 262 -> 214 us;
+// the first launches after a pause are slower, 800-980 and 240-255).  On a bare copy of the loop (3.9e8 pairs): four rows 769 us, two 809,
 // one 923; without the per-row test (the pairs interleaved, 229 VGPRs) 884; at
 // four waves per SIMD 923 (29 spills).
 template <bool TAB>
@@ -927,9 +932,9 @@ __device__ __forceinline__ void nearFly64Tile(const NearTile &tl, const int *__r
 // fly (VALU-bound); the host interleaves the two kinds in block order, so every
 // CU holds both at once and the stream and the arithmetic overlap, and a grid
 // smaller than the tiles strides over them.  Without MIX every tile is computed
-// and has a block of its own: the launch of the default configuration, which
-// needs the registers of the mixed form's other branch (171 against 151 VGPRs)
-// for its third wave per SIMD.  Tiles costliest first (desc).
+// and has a block of its own: the launch of the default configuration, which does
+// without the registers of the mixed form's other branch (157 against 167 VGPRs; three
+// waves per SIMD take up to 168).  Tiles costliest first (desc).
 // TAB: e^{-kappa r} from NearK's table (tab, K.nT entries in dynamic LDS), else from
 // 2^(j/256) (256 entries) and expNeg.  tr: the transposed operator's rows.
 #define MIX64_LDS (2 * NEAR_CHUNK * 8)
@@ -5310,7 +5315,7 @@ static bool buildM2LGrid(fbh_ctx *c) {
   }
   // waves per block (one cube): four when there are few cubes, two from 4,096
   // cubes on, where more cubes in flight per CU pay more than more waves per
-  // cube (317k panels: 212 -> 184 us; 81,920: 63 us either way)
+  // cube (317k panels, FP32: 130 -> 113 us)
   const int ncc = (nmU + 2) & ~1, ngg = (nmU + 1) & ~1, nw = c->nCube >= 4096 ? 2 : 4;
   auto lds = [&](size_t elem) {
     return std::max((size_t)nw * (ncc + ngg) * 2 * elem, (size_t)(K / L) * 64 * 4 * elem);
@@ -5706,8 +5711,8 @@ extern "C" fbh_ctx *fbh_create(double kappa, double eps1, double eps2, int qorde
   // only), interleaved in tile order: a tile streams while the streamed share
   // of the interactions so far stays within the fraction f (FABIPB_NEAR_STREAM;
   // FABIPB_NEAR=stream or fly for all of one kind).  The default computes every
-  // tile: the on-the-fly tiles (two target rows per pass over the staged
-  // sources) outrun the 32-byte coefficient stream, and the far chain's
+  // tile: the on-the-fly tiles (four target rows a wave per pass over the
+  // staged sources) outrun the 32-byte coefficient stream, and the far chain's
   // memory-bound passes overlap them better than they overlap the stream.
   double f = 0.0;
   {
@@ -6370,7 +6375,7 @@ extern "C" int fbh_enable_fp32(fbh_ctx *c) {
   HCK(hipGetLastError());
   HCK(hipStreamSynchronize(c->stream));
   {
-    const char *ep = getenv("FABIPB_NEAR32_PAD_KB");   // occupancy sweeps: LDS held per block beyond its 24 KiB
+    const char *ep = getenv("FABIPB_NEAR32_PAD_KB");   // occupancy sweeps: LDS held per block beyond its 18 KiB
     const int kb = ep ? atoi(ep) : 0;
     c->near32Pad = kb > 0 && kb <= 40 ? (size_t)kb * 1024 : 0;
   }
@@ -7496,7 +7501,7 @@ static int stageCharges(fbh_ctx *c, ChargeSet &s, int nChar, const double *pos, 
   }
   if (uni) {
     int o = 0;
-    for (int a = P; a >= 0; a--)   // the order enFar reads them in
+    for (int a = P; a >= 0; a--)   // the order enFar64 and enFar32 read them in
       for (int b = P - a; b >= 0; b--)
         for (int g3 = P - a - b; g3 >= 0; g3--)
           for (int j = 0; j <= (P - a - b - g3) / 2; j++) dsc.push_back(make_int4(a | b << 8 | g3 << 16, j, 0, o++));

@@ -360,8 +360,9 @@ int fbh_near_timing_read(fbh_ctx *ctx, long long *count, double *ms);
  * [3]=nMom(maxOrder), [4]=nMom(ordMom[depth]), [5]=device bytes held, [6]=M2M/L2L
  * links, [7]=nCube, [8]=interactions with stored coefficients (streamed tiles),
  * [9]=nearfield tiles computed on the fly, [10]=nearfield tiles, [11]=corrected
- * special pairs (0 until the on-the-fly tiles need them), [12]=steps of the M2L
- * term grid (0: the M2L runs from per-lane item lists) */
+ * special pairs (0 until the on-the-fly tiles need them), [12]=steps of the FP32
+ * operator's M2L term grid (0: order 9 or FABIPB_M2L=items, whose M2L runs from
+ * per-lane item lists in both precisions) */
 int fbh_stats(fbh_ctx *ctx, long long *out);
 
 /* the context's stream (hipStream_t), for callers that order their own work on it */
